@@ -1,0 +1,109 @@
+"""One-kernel DCT / DST lines (KK_R2R_*): every form at the sizes where its
+packing, pairing or block edges change, along contiguous and strided axes,
+against scipy's pocketfft. f64 meets the repository's 1e-13 gate, f32 its 1e-5
+gate, and f32 also 16 units of rounding (2^-24) times log2 of the FFT length:
+each stage adds a few units, the phases run in f64."""
+import math
+
+import numpy as np
+import pytest
+
+import vkfft_amd as vk
+from oracle import oracle as o
+
+pytestmark = pytest.mark.gpu
+
+KINDS = ["dct1", "dct2", "dct3", "dct4", "dst1", "dst2", "dst3", "dst4"]
+
+
+def _plan(ctx, name, dims, batch, prec, direction=vk.Direction.Forward, omit=()):
+    t = int(name[-1])
+    kind = vk.TransformKind.dct(t) if name.startswith("dct") else vk.TransformKind.dst(t)
+    c = vk.FftConfig.new(dims).with_batch_count(batch).with_precision(prec).with_transform(kind)
+    for ax in omit:
+        c.with_omit_dimension(ax, True)
+    return vk.TransformIr.build(c, direction)
+
+
+def _check(y, ref, n, prec):
+    err = o.rel_l2(y, ref)
+    assert err <= (1e-13 if prec == vk.Precision.F64 else min(1e-5, 16 * 2.0 ** -24 * math.log2(2 * n))), (n, err)
+
+
+@pytest.mark.parametrize("name", KINDS)
+@pytest.mark.parametrize("prec", [vk.Precision.F32, vk.Precision.F64])
+def test_rows(hip_ctx, name, prec):
+    import scipy.fft as sf
+    f = sf.dct if name.startswith("dct") else sf.dst
+    # smallest, odd and even halves, fixed shapes and the runtime shape (14, 26, 1386), ragged last blocks
+    for n, batch in ((2, 5), (3, 1), (4, 130), (6, 3), (14, 67), (15, 64), (26, 9), (64, 33), (100, 7), (720, 4),
+                     (1000, 3), (1386, 2), (2048, 3), (16384 if prec == vk.Precision.F32 else 8192, 2)):
+        if name == "dct1":
+            n += 1  # the reduction of type I has n - 1 points
+        if name == "dst1":
+            n -= 1
+        if n < 2:
+            continue
+        x = o.uniform(n * batch, n + batch, np.float32 if prec == vk.Precision.F32 else np.float64)
+        ir = _plan(hip_ctx, name, [n], batch, prec)
+        y = hip_ctx.execute_transform(ir, x)
+        _check(y, f(x.astype(np.float64).reshape(batch, n), type=int(name[-1]), axis=-1).reshape(-1), n, prec)
+        labels = [p["kernel"] for p in hip_ctx.plan(ir).describe()["passes"]]
+        odd4 = name.endswith("4") and n % 2
+        assert odd4 or labels == ["r2r_line"], (name, n, labels)
+
+
+@pytest.mark.parametrize("name", KINDS)
+@pytest.mark.parametrize("prec", [vk.Precision.F32, vk.Precision.F64])
+def test_strided_lines(hip_ctx, name, prec):
+    import scipy.fft as sf
+    f = sf.dct if name.startswith("dct") else sf.dst
+    # columns below, at and above the lines of a block, odd column counts, several outer lines
+    for n, inner, batch in ((2, 1, 3), (4, 31, 2), (12, 33, 3), (18, 64, 1), (30, 5, 7), (44, 37, 2), (96, 32, 2),
+                            (720, 65, 1), (2048, 17, 1), (27, 35, 2)):
+        if name == "dct1":
+            n += 1
+        if name == "dst1":
+            n -= 1
+        if n < 2:
+            continue
+        x = o.uniform(n * inner * batch, n + inner, np.float32 if prec == vk.Precision.F32 else np.float64)
+        y = hip_ctx.execute_transform(_plan(hip_ctx, name, [n, inner], batch, prec, omit=(1,)), x)
+        ref = f(x.astype(np.float64).reshape(batch, n, inner), type=int(name[-1]), axis=1).reshape(-1)
+        _check(y, ref, n, prec)
+
+
+@pytest.mark.parametrize("name", ["dct2", "dct3", "dct4", "dct1", "dst2", "dst3"])
+def test_lines_stay_on_their_own(hip_ctx, name):
+    """A line of NaN, of infinities or of tiny values leaves its neighbours
+    bit for bit as they are alone, and a small line keeps its own relative error."""
+    n, batch = 48, 9
+    x = o.uniform(n * batch, 5, np.float32).reshape(batch, n)
+    ir = _plan(hip_ctx, name, [n], batch, vk.Precision.F32)
+    clean = hip_ctx.execute_transform(ir, x.reshape(-1)).reshape(batch, n)
+    bad = x.copy()
+    bad[1], bad[4], bad[6] = np.nan, np.inf, x[6] * np.float32(2.0 ** -60)
+    y = hip_ctx.execute_transform(ir, bad.reshape(-1)).reshape(batch, n)
+    for b in (0, 2, 3, 5, 7, 8):
+        assert np.array_equal(y[b], clean[b]), b
+    assert np.array_equal(y[6], clean[6] * np.float32(2.0 ** -60))
+    assert not np.isfinite(y[1]).any() and not np.isfinite(y[4]).all()
+
+
+@pytest.mark.parametrize("name", KINDS)
+def test_one_kernel_matches_the_three_passes(hip_ctx, name, monkeypatch):
+    """The same plans with VKFX_R2R_FUSED=0 (pre pass, complex FFT, post pass)."""
+    dims, batch = [36, 50], 3
+    x = o.uniform(36 * 50 * batch, 8, np.float64)
+    for direction in (vk.Direction.Forward, vk.Direction.Inverse):
+        ir = _plan(hip_ctx, name, dims, batch, vk.Precision.F64, direction)
+        y = hip_ctx.execute_transform(ir, x)
+        monkeypatch.setenv("VKFX_R2R_FUSED", "0")
+        ctx = vk.HipExecutionContext(0)
+        try:
+            z = ctx.execute_transform(ir, x)
+            assert any(p["kernel"] == "r2r_pre" for p in ctx.plan(ir).describe()["passes"])
+        finally:
+            ctx.close()
+            monkeypatch.delenv("VKFX_R2R_FUSED")
+        assert o.rel_l2(y, z) <= 1e-14

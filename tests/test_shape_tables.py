@@ -67,3 +67,9 @@ def test_recorded_strides_are_model_optimal_for_small_shapes():
             assert round(cur, 3) <= best[0] + 1e-9, (name, it, best)
             checked += 1
     assert checked >= 8
+
+
+@pytest.mark.parametrize("name", ["kf_r2r_f32", "kf_r2r_f64"])
+def test_r2r_tables_match_generator(name):
+    g = _gen()
+    assert open(os.path.join(CSRC, name + ".hip")).read() == g.render(name)

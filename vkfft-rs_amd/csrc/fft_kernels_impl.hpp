@@ -26,6 +26,7 @@
 //   IoFsCBlue     Bluestein column pass: IFFT, chirp multiply, truncate to N
 //   IoBlue1       whole Bluestein transform when the convolution fits LDS
 //   IoConv1       one-upload convolution: FFT, kernel-spectrum multiply, IFFT
+//   IoR2r         DCT / DST line: reorder or phase, half-size FFT, phase or reorder
 //   IoConvB       two-upload convolution row pass: FFT, natural-order
 //                 kernel-spectrum multiply, IFFT, inverse four-step twiddle
 //
@@ -58,14 +59,18 @@ enum Layout : int { LAY_ANY = 0, LAY_ROW = 1, LAY_COL = 2, LAY_STAGED = 3 };
 // IO policies through the same interface.
 struct DynDims {
     static constexpr bool NTI = false, NTO = false;
+    static constexpr bool kFixed = false, COL = false;
+    static constexpr int kN = 0, kTT = 0;
     static __device__ __forceinline__ int N(const KArgs& a) { return a.N; }
     static __device__ __forceinline__ int G(const KArgs& a) { return a.G; }
     static __device__ __forceinline__ int LS(const KArgs& a) { return a.LS; }
     static __device__ __forceinline__ int PS(const KArgs& a) { return a.PS; }
 };
-template <int N_, int G_, int LS_, int PS_, bool NTI_ = false, bool NTO_ = false>
+template <int N_, int G_, int LS_, int PS_, int TT_, bool COL_, bool NTI_ = false, bool NTO_ = false>
 struct FixDims {
     static constexpr bool NTI = NTI_, NTO = NTO_;
+    static constexpr bool kFixed = true, COL = COL_;
+    static constexpr int kN = N_, kTT = TT_;
     static __device__ __forceinline__ constexpr int N(const KArgs&) { return N_; }
     static __device__ __forceinline__ constexpr int G(const KArgs&) { return G_; }
     static __device__ __forceinline__ constexpr int LS(const KArgs&) { return LS_; }
@@ -736,6 +741,10 @@ struct IoC2RHalfEdge : IoC2RHalf {
         staged_store<IoC2RHalfEdge, D, T, S>(a, lds, li, true);
     }
 };
+
+}  // namespace vkfx
+#include "fft_r2r.hpp"
+namespace vkfx {
 
 // Four-step column pass. Line = column n2 of the [N1][N2] view (C = N2);
 // FFT over n1 (length N1); store Y[k1][n2] * W_M^(dir * n2 * k1).
@@ -1758,7 +1767,7 @@ struct Shape {
     static_assert((R * ... * 1) == N_, "radices must multiply to the length");
     static_assert(G_ >= 1 && G_ <= kMaxLinesPerBlock && TT_ >= 1 && G_ * TT_ <= 1024, "block shape");
     using Radices = RList<R...>;
-    using Dims = FixDims<N_, G_, LS_, PS_>;
+    using Dims = FixDims<N_, G_, LS_, PS_, TT_, COL_>;
 };
 
 // LDS slot of element e0 + i*STEP. When STEP is a multiple of the pad period
@@ -2115,7 +2124,7 @@ template <class Base, int W, bool NTIN, bool NTOUT>
 struct Tuned : Base {
     static constexpr int WPE = W;
     static constexpr bool NTI = NTIN, NTO = NTOUT;
-    using Dims = FixDims<Base::N, Base::G, Base::LS, Base::PS, NTIN, NTOUT>;
+    using Dims = FixDims<Base::N, Base::G, Base::LS, Base::PS, Base::TT, Base::COL, NTIN, NTOUT>;
 };
 template <typename T, int S, class IO, class Sh>
 __global__ __launch_bounds__(Sh::G* Sh::TT) __attribute__((amdgpu_waves_per_eu(Sh::WPE > 0 ? Sh::WPE : 1, 8))) void k_fix_occ(
@@ -2146,6 +2155,9 @@ KernelFn pick_dyn(KernelKind kind) {
         case KK_RADER_FFT: return k_dyn<T, S, IoRader, W>;
         case KK_RADER_DIRECT: return k_rader_direct<T>;
         case KK_CONV_1: return k_dyn<T, S, IoConv1, W>;
+        case KK_R2R_II: if constexpr (S < 0) return k_dyn<T, S, IoR2rII, W>; else return nullptr;
+        case KK_R2R_III: if constexpr (S > 0) return k_dyn<T, S, IoR2rIII, W>; else return nullptr;
+        case KK_R2R_MISC: return k_dyn<T, S, IoR2rMisc, W>;
         default: return nullptr;
     }
 }

@@ -704,7 +704,80 @@ HEADS['kf_round_nd_f64'] = HEADS_ROUND_ND.format(p='f64')
 HEADS['kf_round_f32'] = HEADS_ROUND.format(p='f32')
 HEADS['kf_round_f64'] = HEADS_ROUND.format(p='f64')
 
-FUNCS = {'kf_blue_rows_f32': 'fixed_table_blue_rows_f32', 'kf_blue_rows_f64': 'fixed_table_blue_rows_f64',
+
+
+# DCT / DST lines of types II and III (half-size packed FFT of M points, both
+# ends staged through LDS), for the M of the C2C rows above and of the benchmark
+# lengths, and strided lines of every M with factors 2, 3 and 5 up to 1024.
+# Chosen from timed variants (8.4M f32 / 4.2M f64 points, us a pass):
+# - f32 rows keep the C2C shape, except 16-point radices followed by a 3 or 5
+#   (one butterfly of 16 a thread leaves six of the last stage to each): those
+#   take radices up to 8 (M = 640 24.7 -> 21.0, 80 38.0 -> 21.4, 1536 24.7 -> 21.7);
+#   f64 rows take radices up to 8 and M / the smallest radix threads, as the
+#   f64 phases of the ends need more threads in flight (640 27.4 -> 18.7,
+#   1000 23.1 -> 20.1, 512 20.0 -> 17.1).
+# - strided f32 lines: 32 adjacent lines (128-byte segments of reals) while two
+#   blocks fit a CU, else 16, whose 64-byte halves meet in one L2 (neighbouring
+#   groups run on one XCD): M = 360 46.5 -> 35.1, 512 31.4 -> 30.1, 96 27.0
+#   against 30.8; f64 16, else 8 lines and M / the smallest radix threads
+#   (256 31.5 -> 25.5, 512 30.4 -> 27.5).
+def r2r_rows(prec):
+    p, eb = ('f64', 16) if prec else ('f32', 8)
+    src = {}
+    for t in ('kf_pow2_' + p, 'kf_fam_' + p, 'kf_round_' + p, 'kf_round_nd_' + p):
+        for r in TABLES[t]:
+            if not isinstance(r, str) and r[0] == 'PLAIN' and not r[5]:
+                src[r[2]] = r
+    for r in ND_CFG[prec]:
+        if not r[5]:
+            src[r[2]] = r
+    rows = []
+
+    def add(m, tt, G, col, rad, ps, ls):
+        rows.append(('R2R_II', 'R2rII', m, tt, G, col, rad, ps, ls))
+        rows.append(('R2R_III', 'R2rIII', m, tt, G, col, rad, ps, ls))
+
+    for m in sorted(src):
+        _, _, _, tt, G, _, rad, ps, ls = src[m]
+        small = radix_plan(m, (8, 6, 5, 4, 3, 2))
+        if small and (prec or (max(rad) == 16 and m & (m - 1))):
+            rad = small
+            tt = m // (min(rad) if prec else max(rad))
+            while tt > 1024:
+                tt = (tt + 1) // 2
+            ps = 3 if prec else 4
+            ls = m + (m >> ps)
+            ls += 1 - ls % 2
+            G = max(1, min(64, 256 // tt))
+            while G > 1 and G * ls * eb > 80 * 1024:
+                G //= 2
+        add(m, tt, G, False, rad, ps, ls)
+    for m in _smooth(6, 1024):
+        rad = radix_plan(m, (10, 9, 8, 6, 5, 4, 3, 2)) if prec else radix_plan(m)
+        tt = m // (min(rad) if prec else max(rad))
+        ls = m + 1 - m % 2
+        G, low = (16, 8) if prec else (32, 16)
+        while G > low and (G * ls * eb > 80 * 1024 or G * tt > 1024):
+            G //= 2
+        while G > 1 and G * ls * eb > 156 * 1024:
+            G //= 2
+        while G * tt > 1024:
+            tt = (tt + 1) // 2
+        add(m, tt, G, True, rad, 30, ls)
+    return rows
+
+
+TABLES['kf_r2r_f32'] = r2r_rows(0)
+TABLES['kf_r2r_f64'] = r2r_rows(1)
+HEADS_R2R = ("// Fixed shapes of the one-kernel DCT / DST lines of types II and III (even\n"
+             "// lengths 2 M), {p}: rows for the M of the C2C rows, strided lines of every M\n"
+             "// with factors 2, 3 and 5 up to 1024 in blocks of up to 32 (f32) / 16 (f64)\n"
+             "// adjacent lines. Type II runs the forward FFT, type III the inverse.\n")
+HEADS['kf_r2r_f32'] = HEADS_R2R.format(p='f32')
+HEADS['kf_r2r_f64'] = HEADS_R2R.format(p='f64')
+
+FUNCS = {'kf_r2r_f32': 'fixed_table_r2r_f32', 'kf_r2r_f64': 'fixed_table_r2r_f64',
+         'kf_blue_rows_f32': 'fixed_table_blue_rows_f32', 'kf_blue_rows_f64': 'fixed_table_blue_rows_f64',
          'kf_blue_edge_f32': 'fixed_table_blue_edge_f32', 'kf_blue_edge_f64': 'fixed_table_blue_edge_f64',
          'kf_real_edge_f32': 'fixed_table_real_edge_f32', 'kf_real_edge_f64': 'fixed_table_real_edge_f64',
          'kf_plain_edge_f32': 'fixed_table_plain_edge_f32', 'kf_plain_edge_f64': 'fixed_table_plain_edge_f64',
@@ -717,6 +790,8 @@ FUNCS = {'kf_blue_rows_f32': 'fixed_table_blue_rows_f32', 'kf_blue_rows_f64': 'f
 
 def roles(kind, col):
     """(direction, nontemporal input, nontemporal output) registered."""
+    if kind in ("R2R_II", "R2R_III"):
+        return [(-1 if kind == "R2R_II" else 1, not col, col)]
     if kind in ("BLUE_1", "BLUE_1_EDGE"):
         return [(-1, True, True)]
     if kind in ("FS_A", "FS_B"):
@@ -776,7 +851,7 @@ def check():
     for name, items in TABLES.items():
         eb = 16 if name.endswith("f64") else 8
         for it in items:
-            if isinstance(it, str) or it[0] in ("R2C_HALF", "C2R_HALF", "R2C_HALF_EDGE", "C2R_HALF_EDGE"):
+            if isinstance(it, str) or it[0] in ("R2C_HALF", "C2R_HALF", "R2C_HALF_EDGE", "C2R_HALF_EDGE", "R2R_II", "R2R_III"):
                 continue
             kind, io, N, TT, G, col, rad, PS, LS = it
             staged = io == "PlainStaged"

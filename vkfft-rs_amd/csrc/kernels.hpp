@@ -44,6 +44,9 @@ enum KernelKind : int {
     KK_PLAIN_EDGE,     // one-upload 1-D KK_PLAIN rows with storage conversion and zero intervals (fixed shapes only)
     KK_PLAIN_EDGE_IN,  // KK_PLAIN first pass of an N-D chunk reading half-precision storage (fixed shapes only)
     KK_PLAIN_EDGE_OUT, // KK_PLAIN last pass of an N-D chunk writing half-precision storage (fixed shapes only)
+    KK_R2R_II,         // even DCT-II / DST-II line in one kernel: reorder, packed half-size FFT, phase on store
+    KK_R2R_III,        // even DCT-III / DST-III line in one kernel: phase and preprocess, packed half-size FFT, reorder
+    KK_R2R_MISC,       // the other one-kernel DCT / DST forms (types I and IV, odd II / III), by KArgs::rop
     KK_COUNT
 };
 
@@ -136,6 +139,19 @@ struct KArgs {
     // KK_CONV_1 over 1-D lines (C = 1, line = o * C1 + o1): the line's
     // kernel-spectrum plane starts at o * spec_os + o1 * spec_os1
     long long spec_os, spec_os1;
+    // KK_R2R_*: line form (R2rForm) and the DST flag; a line holds nvalid
+    // reals, rlo / rhi / rshift are the two-level f64 table of its phases
+    int rop, rflip;
+};
+
+// Forms of a DCT / DST line in one kernel (KArgs::rop).
+enum R2rForm : int {
+    R2R_F_REORDER = 0,       // even type II: half-size packed FFT
+    R2R_F_SPECTRUM = 1,      // even type III: half-size packed inverse FFT
+    R2R_F_HALF = 2,          // even type IV: half-size FFT of phased pairs
+    R2R_F_SYM = 3,           // type I: half-size packed FFT of the even / odd extension
+    R2R_F_REORDER_FULL = 4,  // odd type II: full-size FFT, zero imaginary part
+    R2R_F_SPECTRUM_FULL = 5  // odd type III: full-size inverse FFT
 };
 
 // Radices up to this are Stockham butterflies; a larger (prime) radix in a

@@ -95,6 +95,27 @@ hipError_t check_launch(KernelKind kind, int prec, int dir, const KArgs& a, unsi
     if ((a.flags & KF_EDGE) && (fixed || kind != KK_PLAIN || (a.flags & KF_DYN_PRE) || a.zl > a.zr || a.zl < 0 ||
                                 a.zr > a.N))
         return hipErrorInvalidConfiguration;
+    // one-kernel DCT / DST lines: nvalid reals whose form has an FFT of N
+    // points, in the form's direction, with the phase table
+    if (kind == KK_R2R_II || kind == KK_R2R_III || kind == KK_R2R_MISC) {
+        const long long n = a.nvalid;
+        long long N = -1;
+        switch (a.rop) {
+            case R2R_F_REORDER:
+            case R2R_F_SPECTRUM:
+            case R2R_F_HALF: N = n % 2 == 0 ? n / 2 : -1; break;
+            case R2R_F_SYM: N = a.rflip ? n + 1 : n - 1; break;
+            case R2R_F_REORDER_FULL:
+            case R2R_F_SPECTRUM_FULL: N = n; break;
+            default: break;
+        }
+        const bool inverse = a.rop == R2R_F_SPECTRUM || a.rop == R2R_F_SPECTRUM_FULL;
+        const bool own = kind == KK_R2R_II    ? a.rop == R2R_F_REORDER
+                         : kind == KK_R2R_III ? a.rop == R2R_F_SPECTRUM
+                                              : a.rop != R2R_F_REORDER && a.rop != R2R_F_SPECTRUM;
+        if (!own || n < 2 || N < 1 || N != a.N || (dir > 0) != inverse || !a.rlo || !a.rhi)
+            return hipErrorInvalidConfiguration;
+    }
     // the register-exchange kernels address contiguous lines (element stride 1)
     if (fixed && fixed->table == FT_WAVE1024 && (a.in_es != 1 || a.out_es != 1 || !a.tw))
         return hipErrorInvalidConfiguration;

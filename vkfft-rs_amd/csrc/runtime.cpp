@@ -2040,18 +2040,67 @@ int plan_r2r(Ctx& c, size_t n, size_t batch, int kind, int dir, bool normalize, 
             }
             break;
     }
-    a.s *= scale;
     const size_t L = (size_t)a.L;
     const bool f64 = c.prec == 1;
     AxisDecision ad = plan_c2c_axis(L, batch, f64, false, c.tuning,
                                     planner_device(p->ctx->profile.shared_memory_bytes));
-    p->full_bytes = std::max(p->full_bytes, batch * L * csize(c.prec));
     p->serial = true;
     static const char* kNames[] = {"dct1", "dct2", "dct3", "dct4", "dst1", "dst2", "dst3", "dst4"};
     c.js << "\"r2r\":{\"type\":\"" << kNames[kind] << "\",\"runs\":\"" << kNames[eff] << "\",\"fft_len\":" << L
          << ",\"c2c\":\""
          << (ad.algorithm == Algorithm::Stockham ? "stockham" : ad.algorithm == Algorithm::Rader ? "rader" : "bluestein")
          << "\"},";
+    // One kernel per line where the packed (even types: half-length) FFT of
+    // the reduction is a Stockham length of one upload; odd type IV, longer
+    // lines and lines whose reduction runs as Rader or Bluestein keep the
+    // pre pass / complex FFT / post pass below. VKFX_R2R_FUSED=0 keeps those
+    // passes everywhere (comparison runs).
+    const char* rf = getenv("VKFX_R2R_FUSED");
+    if (!(rf && rf[0] == '0') && ad.algorithm == Algorithm::Stockham && n >= 2 && !(eff % 4 == 3 && n % 2)) {
+        const bool dst = eff >= 4, even = n % 2 == 0;
+        int form = R2R_F_SYM;
+        size_t N = dst ? n + 1 : n - 1, troot = 2 * N;
+        if (eff % 4 == 1 || eff % 4 == 2) {
+            form = eff % 4 == 1 ? (even ? R2R_F_REORDER : R2R_F_REORDER_FULL)
+                                : (even ? R2R_F_SPECTRUM : R2R_F_SPECTRUM_FULL);
+            N = even ? n / 2 : n;
+            troot = 4 * n;
+        } else if (eff % 4 == 3) {
+            form = R2R_F_HALF;
+            N = n / 2;
+            troot = 8 * n;
+        }
+        const KernelKind kind_r = form == R2R_F_REORDER    ? KK_R2R_II
+                                  : form == R2R_F_SPECTRUM ? KK_R2R_III
+                                                           : KK_R2R_MISC;
+        const bool rows = inner == 1;
+        const Geometry g0 = geometry(N, c.prec, 1, c.lds_max, c.lds_max);
+        // strided lines: 32 (f32) / 16 (f64) adjacent lines, 128-byte segments
+        // of reals; rows: about 256 threads
+        Geometry g = one_upload(N, c.prec, c.lds_max)
+                         ? kernel_geometry(kind_r, c.prec, fft_dir, N, !rows,
+                                           rows ? std::max(1, 256 / g0.TT) : (c.prec ? 16 : 32), c.lds_max,
+                                           rows ? c.lds_budget : c.lds_max)
+                         : Geometry{};
+        if (g.ok) {
+            KArgs k = blank();
+            k.C = (long long)inner;
+            k.in_es = k.out_es = (long long)inner;
+            k.in_cs = k.out_cs = 1;
+            k.in_os = k.out_os = (long long)(n * inner);
+            k.flags = rows ? (KF_IN_ROWMAJOR | KF_OUT_ROWMAJOR) : KF_XCD_GROUPS;
+            k.scale = scale;
+            k.nvalid = (long long)n;
+            k.rop = form;
+            k.rflip = dst ? 1 : 0;
+            int rc = two_level(p, troot, 1, &k.rlo, &k.rhi, &k.rshift);
+            if (rc) return rc;
+            return add_launch(c, kind_r, fft_dir, g, k, (long long)batch, blocks_for(batch, g.G), in_sel, 0, SEL_OUT,
+                              0, "r2r_line");
+        }
+    }
+    a.s *= scale;
+    p->full_bytes = std::max(p->full_bytes, batch * L * csize(c.prec));
     Launch pre{};
     pre.r2r = 1;
     pre.ra = a;
