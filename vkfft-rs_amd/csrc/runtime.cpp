@@ -860,6 +860,7 @@ bool xcd_groups(KernelKind kind) {
 int add_launch(Ctx& c, KernelKind kind, int dir, const Geometry& g, KArgs a, long long nlines, unsigned grid,
                int in_sel, size_t in_off, int out_sel, size_t out_off, const char* label) {
     if (xcd_groups(kind)) a.flags |= KF_XCD_GROUPS;
+    if (const char* e = getenv("VKFX_XCD_GROUPS"); e && e[0] != '1') a.flags &= ~KF_XCD_GROUPS;
     a.N = g.N;
     a.TT = g.TT;
     a.G = g.G;
@@ -1413,6 +1414,24 @@ bool split_strided_axis(size_t len, int prec, size_t lds_budget, size_t* l1, siz
     return true;
 }
 
+// Strided lines whose row segments do not start and end on 128-byte lines of
+// memory (the row pitch of `inner` elements or the block's G elements are not
+// whole lines) share a line with the neighbouring group at both ends of every
+// segment. Their groups are dealt to the XCDs in contiguous ranges, so both
+// halves of a shared line meet in one L2, and they use cached accesses (a
+// nontemporal store writes its part of the line on its own). Aligned segments
+// share nothing and keep the round-robin order (1024^2 x 16: 106 us, 112 in
+// ranges). Measured, us a pass, round-robin and nontemporal against ranges and
+// cached: f32 columns of 512 over rows of 405 36.2 -> 23.8, 360 27.4 -> 18.5,
+// 100 20.6 -> 14.5, 1080 over 961 (16 frames, inverse) 87 -> 63; f64 512 over 405
+// 29.8 -> 25.5; [405, 405, 75] x 2 whole 349 -> 256. The passes of a split axis keep
+// their order: the first (segments along L2 x inner) measured 5-15% slower in
+// ranges, the second 3-10% faster on its own, but the pass that follows it slower
+// by as much (1080 x 1920 frames, inverse: 49 -> 52 and C2R rows 56 -> 65).
+bool shares_lines(size_t inner, int G, int prec) {
+    return (inner * csize(prec)) % 128 != 0 || ((size_t)G * csize(prec)) % 128 != 0;
+}
+
 // Axes whose bit is set in `omit` are left untransformed (the real axis of an
 // N-D real transform).
 int plan_c2c_nd(Ctx& c, const vkfx_plan_desc& d, uint32_t omit) {
@@ -1509,6 +1528,7 @@ int plan_c2c_nd(Ctx& c, const vkfx_plan_desc& d, uint32_t omit) {
                             "N-D axis length " + std::to_string(len) + " exceeds one upload");
             const int want = contiguous ? std::max(1, 256 / g0.TT) : (prec ? 8 : 16);
             Geometry g = kernel_geometry(KK_PLAIN, prec, dir, len, !contiguous, want, c.lds_max, c.lds_budget);
+            if (!contiguous && shares_lines(inner, g.G, prec)) a.flags |= KF_XCD_GROUPS;
             rc = add_launch(c, KK_PLAIN, dir, g, a, lines, blocks_for(lines, g.G), in_sel, off, SEL_OUT, off,
                             contiguous ? "stockham_rows" : "stockham_columns");
         } else {
@@ -1523,6 +1543,7 @@ int plan_c2c_nd(Ctx& c, const vkfx_plan_desc& d, uint32_t omit) {
                 if (g0.ok) {
                     const int want = contiguous ? std::max(1, 256 / g0.TT) : (prec ? 8 : 16);
                     Geometry g = geometry_rader(len, prec, want, c.lds_max, c.lds_budget);
+                    if (!contiguous && shares_lines(inner, g.G, prec)) a.flags |= KF_XCD_GROUPS;
                     note_rader_mixed(c, len, g);
                     return add_launch(c, KK_PLAIN, dir, g, a, lines, blocks_for(lines, g.G), in_sel, off, SEL_OUT,
                                       off, "rader_mixed_axis");
@@ -1539,6 +1560,7 @@ int plan_c2c_nd(Ctx& c, const vkfx_plan_desc& d, uint32_t omit) {
             if (rc) return rc;
             a.chirp = t.chirp, a.spec = t.spec;
             a.nvalid = (long long)len, a.nout = (long long)len, a.M = (long long)M;
+            if (!contiguous && shares_lines(inner, g.G, prec)) a.flags |= KF_XCD_GROUPS;
             rc = add_launch(c, KK_BLUE_1, -1, g, a, lines, blocks_for(lines, g.G), in_sel, off, SEL_OUT, off,
                             "bluestein_axis");
         }
@@ -3143,6 +3165,11 @@ int vkfx_plan_create(vkfx_context* ctx, const vkfx_plan_desc* desc_in, vkfx_plan
         if (!L.fixed) continue;
         bool last = true;
         for (size_t j = i + 1; j < p->launches.size() && last; ++j) last = p->launches[j].chunk != L.chunk;
+        // strided lines that share memory lines with their neighbours (shares_lines)
+        if (L.kind == KK_PLAIN && L.fixed->col && (L.a.flags & KF_XCD_GROUPS)) {
+            L.fixed = fixed_variant(L.fixed, false, false);
+            continue;
+        }
         L.fixed = fixed_variant(L.fixed, L.in_sel == SEL_IN, L.out_sel == SEL_OUT && last);
     }
     // two lanes pay a fork/join (two events, ~10 us) per execute, so only
