@@ -1,0 +1,72 @@
+"""Strided axes of 640 to 1247 points in one pass (kf_cols_*): every registered
+length, ragged last blocks and odd row pitches, and both sides of the rule that
+picks one pass or two, against numpy; the fused axis-0 convolution and the
+mixed-storage last pass on the same shapes."""
+import numpy as np
+import pytest
+
+import vkfft_amd as vk
+from oracle import oracle as o
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = [640, 648, 675, 720, 729, 750, 768, 800, 810, 864, 900, 960, 972, 1000, 1024, 1080, 1125, 1152, 1200, 1215]
+
+
+def _run(ctx, dims, batch, prec, direction):
+    wide = prec == vk.Precision.F64
+    x = o.complex_uniform(int(np.prod(dims)) * batch, dims[0] + batch, np.complex128 if wide else np.complex64)
+    c = vk.FftConfig.new(dims).with_batch_count(batch).with_precision(prec).with_inverse_normalization(True)
+    ir = vk.TransformIr.build(c, direction)
+    y = ctx.execute_transform(ir, x)
+    f = np.fft.fftn if direction == vk.Direction.Forward else np.fft.ifftn
+    ref = f(x.astype(np.complex128).reshape([batch] + dims), axes=tuple(range(1, 1 + len(dims)))).reshape(-1)
+    assert o.rel_l2(y, ref) <= (2e-13 if wide else 2e-6), (dims, batch)
+    return ctx.plan(ir).describe()["passes"]
+
+
+@pytest.mark.parametrize("n", LENGTHS)
+@pytest.mark.parametrize("prec,G", [(vk.Precision.F32, 16), (vk.Precision.F64, 8)])
+def test_lengths(hip_ctx, n, prec, G):
+    for inner, direction in ((3 * G + 1, vk.Direction.Forward), (4 * G, vk.Direction.Inverse)):
+        batch = 100 * G // inner + 1
+        passes = _run(hip_ctx, [n, inner], batch, prec, direction)
+        assert [p["kernel"] for p in passes] == ["stockham_rows", "stockham_columns"], (n, inner)
+        assert passes[1]["fixed_shape"] and passes[1]["lines_per_block"] == G
+
+
+@pytest.mark.parametrize("blocks,split", [(95, True), (96, False), (256, False), (257, True), (307, True), (308, False)])
+def test_rule(hip_ctx, blocks, split):
+    if hip_ctx.device_profile()["compute_units"] != 256:
+        pytest.skip("the rule's sides are stated for 256 CUs")
+    passes = _run(hip_ctx, [720, 16], blocks, vk.Precision.F32, vk.Direction.Forward)
+    assert ("split_axis_pass1" in [p["kernel"] for p in passes]) == split
+
+
+@pytest.mark.parametrize("n,inner,batch", [(768, 33, 40), (1024, 64, 2), (1215, 16, 3)])
+@pytest.mark.parametrize("prec", [vk.Precision.F32, vk.Precision.F64])
+def test_convolution(hip_ctx, n, inner, batch, prec):
+    wide = prec == vk.Precision.F64
+    dt = np.complex128 if wide else np.complex64
+    x = o.complex_uniform(n * inner * batch, 7, dt)
+    k = o.complex_uniform(n * inner, 8, dt)
+    conv = vk.ConvolutionIr.build(vk.FftConfig.new([n, inner]).with_batch_count(batch).with_precision(prec), k)
+    y = hip_ctx.execute_convolution(conv, x)
+    X = np.fft.fftn(x.astype(np.complex128).reshape(batch, n, inner), axes=(1, 2))
+    ref = np.fft.ifftn(X * k.astype(np.complex128).reshape(n, inner), axes=(1, 2)).reshape(-1)
+    assert o.rel_l2(y, ref) <= (2e-13 if wide else 2e-6)
+
+
+@pytest.mark.parametrize("prec,tol", [(vk.Precision.F16StorageF32Compute, 1e-3),
+                                      (vk.Precision.F64ComputeF32Storage, 1e-7)])
+def test_mixed_storage(hip_ctx, prec, tol):
+    n, inner, batch = 960, 48, 40
+    x = o.complex_uniform(n * inner * batch, 9, np.complex64)
+    c = vk.FftConfig.new([n, inner]).with_batch_count(batch).with_precision(prec)
+    ir = vk.TransformIr.build(c, vk.Direction.Forward)
+    y = hip_ctx.execute_transform_f32(ir, x)
+    xs = x
+    if prec == vk.Precision.F16StorageF32Compute:
+        xs = x.real.astype(np.float16).astype(np.float64) + 1j * x.imag.astype(np.float16).astype(np.float64)
+    ref = np.fft.fft2(xs.astype(np.complex128).reshape(batch, n, inner), axes=(1, 2)).reshape(-1)
+    assert o.rel_l2(y, ref) <= tol

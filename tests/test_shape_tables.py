@@ -73,3 +73,9 @@ def test_recorded_strides_are_model_optimal_for_small_shapes():
 def test_r2r_tables_match_generator(name):
     g = _gen()
     assert open(os.path.join(CSRC, name + ".hip")).read() == g.render(name)
+
+
+@pytest.mark.parametrize("name", ["kf_cols_f32", "kf_cols_f64"])
+def test_long_column_tables_match_generator(name):
+    g = _gen()
+    assert open(os.path.join(CSRC, name + ".hip")).read() == g.render(name)

@@ -237,7 +237,6 @@ TABLES = {
         ('PLAIN', 'Plain', 320, 40, 16, True, [8, 8, 5], 30, 321),
         ('PLAIN', 'Plain', 360, 40, 16, True, [8, 9, 5], 30, 361),
         ('PLAIN', 'Plain', 384, 24, 16, True, [16, 8, 3], 30, 385),
-        ('PLAIN', 'Plain', 640, 40, 8, True, [16, 8, 5], 4, 682),
     ],
     "kf_fam_f64": [
         ('PLAIN', 'PlainStaged', 12, 3, 64, False, [4, 3], 4, 19),
@@ -276,7 +275,6 @@ TABLES = {
         ('PLAIN', 'Plain', 320, 40, 8, True, [8, 8, 5], 30, 321),
         ('PLAIN', 'Plain', 360, 40, 8, True, [8, 9, 5], 30, 361),
         ('PLAIN', 'Plain', 384, 24, 8, True, [16, 8, 3], 30, 385),
-        ('PLAIN', 'Plain', 640, 40, 4, True, [16, 8, 5], 4, 682),
     ],
     "kf_real_rows_f32": [
         ('R2C_HALF', 'R2CHalf', 256, 16, 16, False, [16, 16], 4, 271),
@@ -776,7 +774,36 @@ HEADS_R2R = ("// Fixed shapes of the one-kernel DCT / DST lines of types II and 
 HEADS['kf_r2r_f32'] = HEADS_R2R.format(p='f32')
 HEADS['kf_r2r_f64'] = HEADS_R2R.format(p='f64')
 
-FUNCS = {'kf_r2r_f32': 'fixed_table_r2r_f32', 'kf_r2r_f64': 'fixed_table_r2r_f64',
+# Strided axes longer than 640 points in one pass: 16 (f32) / 8 (f64) adjacent
+# lines (128-byte segments) in one block per CU, up to the length whose lines
+# fill the LDS. The radix plan's threads: of 32 to 64 threads a line, the fewest with
+# the fewest elements to handle one after another (a stage gives a thread
+# ceil(N / R / threads) butterflies of R elements). KK_CONV_1: the same shapes for a
+# convolution's axis 0; KK_PLAIN_EDGE_OUT: the last pass of mixed-storage chunks.
+def long_columns(prec, kinds):
+    eb, G = (16, 8) if prec else (8, 16)
+    rows = []
+    for n in _smooth(640, 1247):
+        rad = radix_plan(n)
+        ls = n + 1 - n % 2
+        if G * ls * eb > 156 * 1024:
+            continue
+        lim = 1024 // G
+        tt = min(range(32, min(lim, 64) + 1), key=lambda t: (sum(-(-(n // r) // t) * r for r in rad), t))
+        rows += [(kind, io, n, tt, G, True, rad, 30, ls) for kind, io in kinds]
+    return rows
+
+
+for _prec, _p in ((0, 'f32'), (1, 'f64')):
+    TABLES['kf_cols_' + _p] = long_columns(_prec, [('PLAIN', 'Plain'), ('PLAIN_EDGE_OUT', 'PlainEdgeOut'),
+                                                   ('CONV_1', 'Conv1F')])
+    HEADS['kf_cols_' + _p] = ("// Fixed shapes of strided axes of 640 to 1247 points (factors 2, 3 and 5) in\n"
+                              "// one pass, {p}: {g} adjacent lines (128-byte segments) per block, one block\n"
+                              "// per CU; the plain pass, the last pass of mixed-storage chunks and the\n"
+                              "// convolution of an axis 0.\n").format(p=_p, g=8 if _prec else 16)
+
+FUNCS = {'kf_cols_f32': 'fixed_table_cols_f32', 'kf_cols_f64': 'fixed_table_cols_f64',
+         'kf_r2r_f32': 'fixed_table_r2r_f32', 'kf_r2r_f64': 'fixed_table_r2r_f64',
          'kf_blue_rows_f32': 'fixed_table_blue_rows_f32', 'kf_blue_rows_f64': 'fixed_table_blue_rows_f64',
          'kf_blue_edge_f32': 'fixed_table_blue_edge_f32', 'kf_blue_edge_f64': 'fixed_table_blue_edge_f64',
          'kf_real_edge_f32': 'fixed_table_real_edge_f32', 'kf_real_edge_f64': 'fixed_table_real_edge_f64',
@@ -790,6 +817,8 @@ FUNCS = {'kf_r2r_f32': 'fixed_table_r2r_f32', 'kf_r2r_f64': 'fixed_table_r2r_f64
 
 def roles(kind, col):
     """(direction, nontemporal input, nontemporal output) registered."""
+    if kind == "CONV_1":
+        return [(-1, False, False)]
     if kind in ("R2R_II", "R2R_III"):
         return [(-1 if kind == "R2R_II" else 1, not col, col)]
     if kind in ("BLUE_1", "BLUE_1_EDGE"):

@@ -39,6 +39,8 @@ const FixedKernel* fixed_table_blue_rows_f64(int* count);
 const FixedKernel* fixed_table_conv(int* count);
 const FixedKernel* fixed_table_fs_edge(int* count);
 const FixedKernel* fixed_table_conv1(int* count);
+const FixedKernel* fixed_table_cols_f32(int* count);
+const FixedKernel* fixed_table_cols_f64(int* count);
 const FixedKernel* fixed_table_r2r_f32(int* count);
 const FixedKernel* fixed_table_r2r_f64(int* count);
 const FixedKernel* fixed_table_blue_edge_f32(int* count);
@@ -72,7 +74,8 @@ static const FixedKernel* registry(int* count) {
                                                 fixed_table_real_edge_f64, fixed_table_plain_edge_f32,
                                                 fixed_table_plain_edge_f64, fixed_table_nd_edge_f32,
                                                 fixed_table_nd_edge_f64, fixed_table_r2r_f32,
-                                                fixed_table_r2r_f64};
+                                                fixed_table_r2r_f64, fixed_table_cols_f32,
+                                                fixed_table_cols_f64};
         constexpr int kTables = (int)(sizeof(tables) / sizeof(tables[0]));
         int counts[kTables], sum = 0;
         const FixedKernel* ptrs[kTables];

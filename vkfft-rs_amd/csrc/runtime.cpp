@@ -1392,10 +1392,30 @@ int plan_c2c_1d(Ctx& c, size_t n, size_t batch, int dir, bool normalize, Algorit
 // columns per block (narrow HBM segments, one block per CU) is split into two
 // passes of length L1 x L2 = len over 32-column tiles: FFT over n1 with the
 // W_len^(n2*k1) twiddle, then FFT over n2 with a natural-order store.
-bool split_strided_axis(size_t len, int prec, size_t lds_budget, size_t* l1, size_t* l2) {
+// One pass instead where a fixed shape of the length moves 128-byte segments
+// (one block per CU: 16 f32 or 8 f64 lines) and its blocks fill the CUs well
+// enough: at least 96 of them (fewer leave CUs idle while each block runs its
+// whole line: 1024 x 1024 f32, 64 blocks, 18.6 us against 17.0 split; 720 x 1280,
+// 80 blocks, 18.3 against 20.2; 1080 x 405 x 4, 102 blocks, 28.4 against 29.0) and no
+// second round that is mostly empty (800 x 800 x 3 f64, 300 blocks on 256 CUs,
+// 38.1 against 36.4; 720 x 1280 x 4, 320 blocks, 38.0 against 37.6). Measured, us,
+// split against one pass: f32 1024 x 1024 x 16 136 -> 107, 1200 x 1280 x 16 202 -> 163,
+// f64 1024 x 1024 x 8 132 -> 101, 1080 x 1280 x 8 186 -> 155. Longer axes stay split:
+// 8 f32 lines of 2048 (64-byte segments) took 88 us against 46 + 39.
+bool split_strided_axis(const Ctx& c, size_t len, size_t lines, size_t* l1, size_t* l2) {
+    const int prec = c.prec;
+    const size_t lds_budget = c.lds_budget;
     const size_t cs = csize(prec);
     const size_t want_cols = prec ? 8 : 16;
     if (len * want_cols * cs <= lds_budget) return false;
+    if (lds_budget >= 80 * 1024 && len <= (1u << 20)) {
+        const FixedKernel* f = find_fixed(KK_PLAIN, prec, -1, (int)len, true);
+        if (f && (size_t)f->G * cs >= 128 && (size_t)f->G * f->LS * cs <= c.lds_max) {
+            const size_t blocks = (lines + f->G - 1) / f->G, cus = c.p->ctx->profile.compute_units;
+            const size_t rounds = cus ? (blocks + cus - 1) / cus : 1;
+            if (blocks >= 96 && (rounds <= 1 || 5 * blocks >= 3 * rounds * cus)) return false;
+        }
+    }
     size_t best1 = 0, best2 = 0, bestmax = SIZE_MAX;
     for (size_t a = 2; a * a <= len; ++a) {
         if (len % a) continue;
@@ -1445,19 +1465,12 @@ int plan_c2c_nd(Ctx& c, const vkfx_plan_desc& d, uint32_t omit) {
     size_t chunk = d.batch;
     bool any_split = false;
     auto active = [&](uint32_t ax) { return d.dims[ax] > 1 && !(omit >> ax & 1u); };
-    for (uint32_t ax = 0; ax + 1 < d.rank; ++ax) {
-        size_t l1, l2;
-        if (d.axis_algorithm[ax] == VKFX_ALG_STOCKHAM && active(ax) &&
-            split_strided_axis(d.dims[ax], prec, c.lds_budget, &l1, &l2))
-            any_split = true;
-    }
     // batch chunks of 128 MB (C3: one 4096^2 f32 image in flight, 2.04 ms per
     // step against 2.40 ms with 256 MB); slab chunks of 256 MB (C4: 2.32 ms
     // against 2.40 ms at 128 MB and 2.47-2.54 ms at 384 MB and above)
     size_t chunk_budget = 128ull << 20, slab_budget = 256ull << 20;
     if (const char* e = getenv("VKFX_ND_CHUNK_MB")) chunk_budget = slab_budget = (size_t)atoll(e) << 20;
     chunk = std::max<size_t>(1, std::min(d.batch, chunk_budget / std::max<size_t>(per_batch * cs, 1)));
-    if (any_split) c.p->work_bytes = std::max(c.p->work_bytes, chunk * per_batch * cs);
     // A volume larger than the chunk budget runs its axes 1.. (which stay
     // inside one slab of fixed index along axis 0) slab chunk by slab chunk,
     // then axis 0 over the whole volume.
@@ -1468,6 +1481,18 @@ int plan_c2c_nd(Ctx& c, const vkfx_plan_desc& d, uint32_t omit) {
     if (chunk == 1 && per_batch * cs > chunk_budget && active(0) && slab_axes >= 2)
         slabs = std::max<size_t>(1, slab_budget / (slab * cs));
     c.js << "\"nd\":{\"chunk\":" << chunk << ",\"slabs_per_chunk\":" << slabs << "},";
+    // whether a strided axis is split, from the elements of a full chunk (the
+    // same for a shorter last chunk)
+    auto split_axis = [&](uint32_t ax, size_t* l1, size_t* l2) {
+        if (d.axis_algorithm[ax] != VKFX_ALG_STOCKHAM || ax + 1 == d.rank) return false;
+        const size_t elems = slabs && ax > 0 ? std::min(slabs, (size_t)d.dims[0]) * slab : chunk * per_batch;
+        return split_strided_axis(c, d.dims[ax], elems / d.dims[ax], l1, l2);
+    };
+    for (uint32_t ax = 0; ax + 1 < d.rank; ++ax) {
+        size_t l1, l2;
+        if (active(ax) && split_axis(ax, &l1, &l2)) any_split = true;
+    }
+    if (any_split) c.p->work_bytes = std::max(c.p->work_bytes, chunk * per_batch * cs);
 
     // Launches of one axis over `total` elements at byte offset `off`.
     auto axis_pass = [&](int ax, size_t total, size_t off, int in_sel) -> int {
@@ -1480,7 +1505,7 @@ int plan_c2c_nd(Ctx& c, const vkfx_plan_desc& d, uint32_t omit) {
         const int alg = d.axis_algorithm[ax];
         int rc;
         size_t l1 = 0, l2 = 0;
-        if (alg == VKFX_ALG_STOCKHAM && !contiguous && split_strided_axis(len, prec, c.lds_budget, &l1, &l2)) {
+        if (alg == VKFX_ALG_STOCKHAM && !contiguous && split_axis((uint32_t)ax, &l1, &l2)) {
             // pass A: lines (o, n2, c), FFT over n1 at stride L2*inner, twiddle, store in place pattern
             Geometry ga = kernel_geometry(KK_FS_A, prec, dir, l1, true, prec ? 8 : 16, c.lds_max, c.lds_budget);
             Geometry gb = kernel_geometry(KK_PLAIN, prec, dir, l2, true, prec ? 8 : 16, c.lds_max, c.lds_budget);
@@ -1962,11 +1987,13 @@ int plan_convolution(Ctx& c, const vkfx_plan_desc& d, size_t coords, size_t out_
     for (uint32_t i = 0; nd_fused && i < d.rank; ++i) nd_fused = d.axis_algorithm[i] == VKFX_ALG_STOCKHAM;
     if (nd_fused) {
         const size_t n0 = d.dims[0], rest = T / n0;
-        const bool split = split_strided_axis(n0, c.prec, c.lds_budget, &sl1, &sl2);
+        const bool split = split_strided_axis(c, n0, d.batch * rest, &sl1, &sl2);
         Geometry g = kernel_geometry(KK_CONV_1, c.prec, -1, n0, true, c.prec ? 8 : 16, c.lds_max, c.lds_budget);
         // strided columns: at least 8 adjacent columns per block, so each
         // HBM access moves 64 bytes or more
-        if (g.ok && g.G >= 8 && (g.fixed || split)) {
+        // and in f64 only where the plain plan takes one pass (a split axis has
+        // too few lines to fill the CUs with whole columns)
+        if (g.ok && g.G >= 8 && (split ? !c.prec : g.fixed != nullptr)) {
             c.js << ",\"fused\":true,\"fused_axis\":0},";
             int rc = transform(d.batch, -1, false, SEL_IN, SEL_FULL, 1u);
             if (rc) return rc;
@@ -1979,6 +2006,7 @@ int plan_convolution(Ctx& c, const vkfx_plan_desc& d, size_t coords, size_t out_
             a.flags = (ca.conj_seq ? KF_CONV_CONJ : 0) | (ca.cross_norm ? KF_CONV_CROSS : 0);
             a.scale = 1.0 / (double)n0;
             a.spec = kernel;
+            if (shares_lines(rest, g.G, c.prec)) a.flags |= KF_XCD_GROUPS;
             const long long lines = (long long)(d.batch * rest);
             rc = add_launch(c, KK_CONV_1, -1, g, a, lines, blocks_for(lines, g.G), SEL_FULL, 0, SEL_OUT, 0,
                             "convolution_fused_axis0");
