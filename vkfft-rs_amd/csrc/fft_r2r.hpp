@@ -70,52 +70,13 @@ __device__ __forceinline__ T& r2r_slot(cpx<T>* line, int m, int ps) {
 // Makhoul's order: v[m] = x[2m] for m < ceil(n/2), else x[2(n-1-m)+1].
 __device__ __forceinline__ int r2r_makhoul_pos(int j, int n) { return (j & 1) ? n - 1 - (j >> 1) : (j >> 1); }
 
-// Items e < count of every line of the block: v = load(line info, e), then
-// use(line info, line index, e, v). Fixed shapes with at least 16 threads a row
-// (64 contiguous bytes) and all strided ones visit the thread's own line,
-// e = t, t + TT, ...: the line's placement is read once, the trip count is a
-// compile-time constant, and U loads are in flight before the first use.
-// Short rows and the runtime shapes walk the block's elements in address order.
-// Lines past the end read line 0 (in bounds) and are never stored.
-// count: CN elements of a fixed shape, `n` of a runtime one.
-template <class D>
-constexpr bool r2r_own_line() {
-    return D::kFixed && (D::COL || D::kTT >= 16);
-}
-template <class D, int CN, int U, class Ld, class Us>
-__device__ __forceinline__ void r2r_visit(const KArgs& a, const LineInfo* li, int n, bool row, Ld&& load, Us&& use) {
-    if constexpr (r2r_own_line<D>()) {
-        constexpr int TT = D::kTT, J = (CN + TT - 1) / TT;
-        const int tid = (int)threadIdx.x;
-        const int g = D::COL ? tid % D::G(a) : tid / TT, t = D::COL ? tid / D::G(a) : tid % TT;
-        const LineInfo L = li[g];
-        using V = decltype(load(L, 0));
-#pragma unroll
-        for (int j0 = 0; j0 < J; j0 += U) {
-            V v[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int e = t + (j0 + u) * TT;
-                if (j0 + u < J && ((j0 + u + 1) * TT <= CN || e < CN)) v[u] = load(L, e);
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int e = t + (j0 + u) * TT;
-                if (j0 + u < J && ((j0 + u + 1) * TT <= CN || e < CN)) use(L, g, e, v[u]);
-            }
-        }
-    } else {
-        coop_for(D::G(a), n, row, [&](int g, int e) { use(li[g], g, e, load(li[g], e)); });
-    }
-}
-
 // exp(-2 pi i k / L) for the k a thread visits. f32 lines of own-line shapes
 // advance it by one f64 multiplication a visit (k grows by TT; the error of the
 // at most 64 steps stays below 2^-45); f64 lines and the other shapes read
 // the table at every k.
 template <typename T, class D>
 struct R2rPhase {
-    static constexpr bool kStep = r2r_own_line<D>() && sizeof(T) == 4;
+    static constexpr bool kStep = own_line<D>() && sizeof(T) == 4;
     cpx<double> w, step;
     __device__ __forceinline__ R2rPhase(const KArgs& a) {
         if constexpr (kStep) {
@@ -155,7 +116,7 @@ struct IoR2rII : IoPlain {
         const T* in = (const T*)a.in;
         const long long es = a.in_es;
         // reals 2i and 2i+1 of the line are v[i] and v[n-1-i]
-        r2r_visit<D, D::kN, 8>(
+        visit_lines<D, D::kN, 8>(
             a, li, D::N(a), row,
             [&](const LineInfo& L, int i) {
                 const T* p = in + L.ib + 2 * (long long)i * es;
@@ -176,7 +137,7 @@ struct IoR2rII : IoPlain {
         const long long es = a.out_es;
         const double sc = a.scale;
         R2rPhase<T, D> phase(a);
-        r2r_visit<D, D::kN / 2 + 1, 1>(
+        visit_lines<D, D::kN / 2 + 1, 1>(
             a, li, M / 2 + 1, row, [&](const LineInfo&, int) { return 0; },
             [&](const LineInfo& L, int g, int k, int) {
                 cpx<double> w, W;
@@ -221,7 +182,7 @@ struct IoR2rIII : IoPlain {
         const T* in = (const T*)a.in;
         const long long es = a.in_es;
         R2rPhase<T, D> phase(a);
-        r2r_visit<D, D::kN / 2 + 1, 4>(
+        visit_lines<D, D::kN / 2 + 1, 4>(
             a, li, M / 2 + 1, row,
             [&](const LineInfo& L, int k) {
                 const T* p = in + L.ib;
@@ -250,7 +211,7 @@ struct IoR2rIII : IoPlain {
         T* out = (T*)a.out;
         const long long es = a.out_es;
         const double sc = a.scale;
-        r2r_visit<D, D::kN, 1>(
+        visit_lines<D, D::kN, 1>(
             a, li, D::N(a), row, [&](const LineInfo&, int) { return 0; },
             [&](const LineInfo& L, int g, int i, int) {
                 if (!L.valid) return;
