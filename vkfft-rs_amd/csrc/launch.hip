@@ -2,10 +2,13 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
 
+#include <algorithm>
 #include <cstdlib>
 #include <map>
 #include <mutex>
 #include <string>
+#include <unordered_map>
+#include <vector>
 
 #include "kernels.hpp"
 
@@ -54,11 +57,24 @@ const FixedKernel* fixed_table_nd_edge_f64(int* count);
 
 // All registered fixed-shape instantiations, merged once (thread-safe
 // static initialisation).
-static const FixedKernel* registry(int* count) {
-    struct Merged {
-        const FixedKernel* all;
-        int total;
-    };
+// Entries are found through `at`: the positions of each (kind, precision,
+// direction, length, lane mapping) in registration order. A plan looks its
+// shapes up several times, and a scan of all entries was the larger part of a
+// small plan's creation.
+struct Merged {
+    const FixedKernel* all;
+    std::unordered_map<uint64_t, std::vector<int>> at;
+    static uint64_t key(int kind, int prec, int dir, int N, bool col) {
+        return ((((uint64_t)(unsigned)N * KK_COUNT + (unsigned)kind) * 2 + (prec ? 1 : 0)) * 2 + (dir > 0 ? 1 : 0)) * 2 +
+               (col ? 1 : 0);
+    }
+    const std::vector<int>& find(int kind, int prec, int dir, int N, bool col) const {
+        static const std::vector<int> none;
+        const auto it = at.find(key(kind, prec, dir, N, col));
+        return it == at.end() ? none : it->second;
+    }
+};
+static const Merged& registry() {
     static const Merged m = [] {
         const FixedKernel* (*tables[])(int*) = {fixed_table_plain, fixed_table_wave, fixed_table_real, fixed_table_blue,
                                                 fixed_table_nd, fixed_table_pow2_f32, fixed_table_pow2_f64,
@@ -93,10 +109,12 @@ static const FixedKernel* registry(int* count) {
                 merged[k].nst = n;
                 ++k;
             }
-        return Merged{merged, sum};
+        Merged out{merged, {}};
+        for (int i = 0; i < sum; ++i)
+            out.at[Merged::key(merged[i].kind, merged[i].prec, merged[i].dir, merged[i].N, merged[i].col)].push_back(i);
+        return out;
     }();
-    *count = m.total;
-    return m.all;
+    return m;
 }
 
 const FixedKernel* find_fixed(KernelKind kind, int prec, int dir, int N, bool col) {
@@ -104,48 +122,33 @@ const FixedKernel* find_fixed(KernelKind kind, int prec, int dir, int N, bool co
     // may build plans under different settings (tests do)
     const char* dis = getenv("VKFX_DISABLE_FIXED");
     if (dis && dis[0] == '1') return nullptr;
-    int total = 0;
-    const FixedKernel* all = registry(&total);
+    const Merged& reg = registry();
+    const std::vector<int>& at = reg.find(kind, prec, dir, N, col);
+    if (at.empty()) return nullptr;
     // VKFX_REGISTER_EXCHANGE=1 prefers the register-exchange shape of a key
     // (one wave per line, no LDS) where one is registered.
     const char* rx = getenv("VKFX_REGISTER_EXCHANGE");
     if (rx && rx[0] == '1')
-        for (int i = 0; i < total; ++i) {
-            const FixedKernel& f = all[i];
-            if (f.kind == kind && f.prec == prec && f.dir == dir && f.N == N && f.col == col &&
-                f.table == FT_WAVE1024)
-                return &f;
-        }
+        for (int i : at)
+            if (reg.all[i].table == FT_WAVE1024) return &reg.all[i];
     // VKFX_FIXED_PICK=k selects the k-th registered variant of a shape key,
     // or its last one if it has fewer (tuning runs); the default is the first.
     // VKFX_FIXED_PICK_K<kind>=k does the same for one KernelKind only.
     const char* pa = getenv("VKFX_FIXED_PICK");
-    const int pick_all = pa ? atoi(pa) : 0;
-    int pick = pick_all;
+    size_t pick = pa ? (size_t)std::max(0, atoi(pa)) : 0;
     if (kind >= 0 && kind < KK_COUNT) {
         const std::string name = "VKFX_FIXED_PICK_K" + std::to_string((int)kind);
-        if (const char* e = getenv(name.c_str())) pick = atoi(e);
+        if (const char* e = getenv(name.c_str())) pick = (size_t)std::max(0, atoi(e));
     }
-    const FixedKernel* last = nullptr;
-    int seen = 0;
-    for (int i = 0; i < total; ++i) {
-        const FixedKernel& f = all[i];
-        if (f.kind == kind && f.prec == prec && f.dir == dir && f.N == N && f.col == col) {
-            last = &f;
-            if (seen++ == pick) return &f;
-        }
-    }
-    return last;
+    return &reg.all[at[std::min(pick, at.size() - 1)]];
 }
 
 const FixedKernel* fixed_variant(const FixedKernel* f, bool nti, bool nto) {
     if (!f || (f->nti == nti && f->nto == nto)) return f;
-    int total = 0;
-    const FixedKernel* all = registry(&total);
-    for (int i = 0; i < total; ++i) {
-        const FixedKernel& v = all[i];
-        if (v.kind != f->kind || v.prec != f->prec || v.dir != f->dir || v.N != f->N || v.col != f->col ||
-            v.TT != f->TT || v.G != f->G || v.PS != f->PS || v.LS != f->LS || v.nst != f->nst || v.nti != nti ||
+    const Merged& reg = registry();
+    for (int i : reg.find(f->kind, f->prec, f->dir, f->N, f->col)) {
+        const FixedKernel& v = reg.all[i];
+        if (v.TT != f->TT || v.G != f->G || v.PS != f->PS || v.LS != f->LS || v.nst != f->nst || v.nti != nti ||
             v.nto != nto || v.table != f->table || v.lds_mult != f->lds_mult)
             continue;
         bool same = true;
@@ -157,12 +160,10 @@ const FixedKernel* fixed_variant(const FixedKernel* f, bool nti, bool nto) {
 
 const FixedKernel* kind_variant(const FixedKernel* f, KernelKind kind) {
     if (!f) return nullptr;
-    int total = 0;
-    const FixedKernel* all = registry(&total);
-    for (int i = 0; i < total; ++i) {
-        const FixedKernel& v = all[i];
-        if (v.kind != kind || v.prec != f->prec || v.dir != f->dir || v.N != f->N || v.col != f->col ||
-            v.TT != f->TT || v.G != f->G || v.PS != f->PS || v.LS != f->LS || v.nst != f->nst ||
+    const Merged& reg = registry();
+    for (int i : reg.find(kind, f->prec, f->dir, f->N, f->col)) {
+        const FixedKernel& v = reg.all[i];
+        if (v.TT != f->TT || v.G != f->G || v.PS != f->PS || v.LS != f->LS || v.nst != f->nst ||
             v.table != f->table || v.lds_mult != f->lds_mult)
             continue;
         bool same = true;
