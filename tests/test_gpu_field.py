@@ -1,0 +1,59 @@
+"""Small 2-D and 3-D complex fields in one kernel: every radix and the shapes at
+the edges of its rules (shortest axes, copied-in first stage, several fields a
+block with a ragged last one, the largest fields and the first that keep the axis
+passes), against numpy and against the axis passes; in place and out of place."""
+import numpy as np
+import pytest
+
+import vkfft_amd as vk
+from oracle import oracle as o
+
+pytestmark = pytest.mark.gpu
+
+# (dims, batch, one kernel in f32, in f64)
+CASES = [([2, 2], 1, True, True), ([2, 2], 3001, True, True), ([3, 5], 2000, True, True), ([64, 64], 1, True, False),
+         ([64, 64], 3, True, False), ([32, 32], 4099, True, True), ([13, 11], 1500, True, True), ([9, 7], 1, True, True),
+         ([16, 16], 5, True, True), ([2, 1000], 2, True, True), ([1000, 2], 2, True, True), ([16, 8, 8], 700, True, True),
+         ([10, 12, 15], 3, True, True), ([3, 2, 26], 4, True, True), ([49, 81], 2, True, True), ([44, 104], 2, True, False),
+         ([16, 16, 16], 2, True, True), ([8, 512], 2, True, True), ([72, 72], 1, True, False), ([91, 77], 512, True, False),
+         ([91, 77], 513, False, False), ([128, 128], 1, False, False), ([36, 60], 2912, True, True), ([36, 60], 2913, False, True),
+         ([17, 16], 2, False, False), ([16, 1], 2, False, False)]
+
+
+def _plan(ctx, dims, batch, prec, direction):
+    c = vk.FftConfig.new(dims).with_batch_count(batch).with_precision(prec).with_inverse_normalization(True)
+    return vk.TransformIr.build(c, direction)
+
+
+@pytest.mark.parametrize("dims,batch,one32,one64", CASES)
+@pytest.mark.parametrize("prec", [vk.Precision.F32, vk.Precision.F64])
+def test_fields(hip_ctx, monkeypatch, dims, batch, one32, one64, prec):
+    wide = prec == vk.Precision.F64
+    x = o.complex_uniform(int(np.prod(dims)) * batch, 5, np.complex128 if wide else np.complex64)
+    axes = tuple(range(1, len(dims) + 1))
+    # the axis passes' bound at these lengths: a few roundings a stage
+    tol = 4e-15 if wide else 1e-6
+    for direction, f in ((vk.Direction.Forward, np.fft.fftn), (vk.Direction.Inverse, np.fft.ifftn)):
+        ir = _plan(hip_ctx, dims, batch, prec, direction)
+        y = hip_ctx.execute_transform(ir, x)
+        ref = f(x.astype(np.complex128).reshape([batch] + dims), axes=axes).reshape(-1)
+        assert o.rel_l2(y, ref) <= tol, (dims, batch, direction)
+        assert ([p["kernel"] for p in hip_ctx.plan(ir).describe()["passes"]] == ["field"]) == (one64 if wide else one32)
+    monkeypatch.setenv("VKFX_FIELD", "0")
+    other = vk.Plan(hip_ctx, ir)
+    assert all(p["kernel"] != "field" for p in other.describe()["passes"])
+
+
+@pytest.mark.parametrize("dims,batch", [([64, 64], 2), ([30, 14], 1100), ([8, 9, 10], 7)])
+def test_in_place(hip_ctx, dims, batch):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.view_as_complex(torch.rand([batch] + dims + [2], generator=g, device="cuda").sub_(0.5))
+    plan = vk.Plan(hip_ctx, _plan(hip_ctx, dims, batch, vk.Precision.F32, vk.Direction.Forward))
+    ref = torch.fft.fftn(x.to(torch.complex128), dim=tuple(range(1, len(dims) + 1)))
+    y = torch.empty_like(x)
+    plan.execute_tensors(x, y)
+    plan.execute_tensors(x, x)
+    torch.cuda.synchronize()
+    assert torch.equal(x, y)
+    assert float((x - ref).abs().norm() / ref.abs().norm()) <= 1e-6

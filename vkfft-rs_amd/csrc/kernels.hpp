@@ -18,6 +18,12 @@ hipError_t static_scratch_address(int device, void** out);
 
 // Kernel families. Each is one HBM pass over its lines; see the comments on
 // the IO policies in fft_kernels.hip for what each one loads and stores.
+#ifdef __HIPCC__
+#define VKFX_HD __host__ __device__
+#else
+#define VKFX_HD
+#endif
+
 enum KernelKind : int {
     KK_PLAIN = 0,      // C2C lines along any axis, scale on store
     KK_R2C_FULL,       // odd-length R2C: real -> complex FFT, keep n/2+1
@@ -47,6 +53,7 @@ enum KernelKind : int {
     KK_R2R_II,         // even DCT-II / DST-II line in one kernel: reorder, packed half-size FFT, phase on store
     KK_R2R_III,        // even DCT-III / DST-III line in one kernel: phase and preprocess, packed half-size FFT, reorder
     KK_R2R_MISC,       // the other one-kernel DCT / DST forms (types I and IV, odd II / III), by KArgs::rop
+    KK_FIELD,          // small 2-D / 3-D complex fields in one kernel (fft_field.hpp)
     KK_COUNT
 };
 
@@ -80,6 +87,8 @@ enum KFlags : int {
     // through the M x M kernel matrix (symmetric planes with KF_CONV_SYM)
     KF_CONV_MATRIX = 65536,
     KF_CONV_SYM = 131072,
+    KF_FIELD_COPY = 262144,  // KK_FIELD: a coalesced copy to LDS before the first stage
+    KF_FIELD_LARGE = 524288,  // KK_FIELD: a radix above 10
 };
 
 // Butterflies per thread in one radix-R stage of the runtime-shape kernel
@@ -143,6 +152,19 @@ struct KArgs {
     // reals, rlo / rhi / rshift are the two-level f64 table of its phases
     int rop, rflip;
 };
+
+// KK_FIELD: length, stages and roots of each axis, last axis first (unused axes:
+// length 1, no stages), and the fields per block; LS spans both LDS buffers. They
+// take places of the Rader and Bluestein arguments, so that every launch's
+// arguments stay as short as they are.
+inline VKFX_HD int& field_dim(KArgs& a, int ax) { return a.roff[ax]; }
+inline VKFX_HD int field_dim(const KArgs& a, int ax) { return a.roff[ax]; }
+inline VKFX_HD int& field_stages(KArgs& a, int ax) { return a.roff[3 + ax]; }
+inline VKFX_HD int field_stages(const KArgs& a, int ax) { return a.roff[3 + ax]; }
+inline VKFX_HD int& field_pack(KArgs& a) { return a.roff[6]; }
+inline VKFX_HD int field_pack(const KArgs& a) { return a.roff[6]; }
+inline VKFX_HD const void*& field_roots(KArgs& a, int ax) { return ax == 0 ? a.chirp : ax == 1 ? a.spec : a.tlo; }
+inline VKFX_HD const void* field_roots(const KArgs& a, int ax) { return ax == 0 ? a.chirp : ax == 1 ? a.spec : a.tlo; }
 
 // Forms of a DCT / DST line in one kernel (KArgs::rop).
 enum R2rForm : int {

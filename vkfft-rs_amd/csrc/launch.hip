@@ -188,7 +188,12 @@ static int lds_limit_bytes() {
 
 size_t max_lds_bytes() { return (size_t)lds_limit_bytes(); }
 
+KernelFn pick_field_f32(int dir, bool large);
+KernelFn pick_field_f64(int dir, bool large);
+
 static KernelFn pick_kernel(KernelKind kind, int prec, int dir, int flags) {
+    if (kind == KK_FIELD)
+        return prec ? pick_field_f64(dir, (flags & KF_FIELD_LARGE) != 0) : pick_field_f32(dir, (flags & KF_FIELD_LARGE) != 0);
     const bool wide = (flags & KF_DYN_WIDE) != 0;
     const int direct = (flags & KF_DYN_DIRECT) ? ((flags & KF_DYN_PRE) ? 2 : 1) : 0;
     const int edge =

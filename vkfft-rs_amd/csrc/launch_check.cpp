@@ -116,6 +116,29 @@ hipError_t check_launch(KernelKind kind, int prec, int dir, const KArgs& a, unsi
         if (!own || n < 2 || N < 1 || N != a.N || (dir > 0) != inverse || !a.rlo || !a.rhi)
             return hipErrorInvalidConfiguration;
     }
+    // fields: the axes' radices multiply to their lengths, the lengths to N; both
+    // buffers hold the block's padded elements, whose indices stay below 2^16
+    if (kind == KK_FIELD) {
+        if (fixed || field_pack(a) < 1 || a.N < 4 || a.N > 65535 / field_pack(a) || a.G != 1) return hipErrorInvalidConfiguration;
+        long long total = 1;
+        int s = 0;
+        for (int ax = 0; ax < 3; ++ax) {
+            if (field_dim(a, ax) < 1 || field_stages(a, ax) < 0 || s + field_stages(a, ax) > a.nstages) return hipErrorInvalidConfiguration;
+            long long n = 1;
+            for (int j = 0; j < field_stages(a, ax); ++j) {
+                const int r = a.radix[s++];
+                if (r < 2 || r > kMaxStockhamRadix || r == 14 || r == 15)
+                    return hipErrorInvalidConfiguration;
+                if (r > 10 && (!(a.flags & KF_FIELD_LARGE) || (prec && r == 12))) return hipErrorInvalidConfiguration;
+                n *= r;
+            }
+            if (n != field_dim(a, ax) || (n > 1 && !field_roots(a, ax))) return hipErrorInvalidConfiguration;
+            total *= n;
+        }
+        const long long points = (long long)a.N * field_pack(a);
+        if (total != a.N || s != a.nstages || a.LS % 2 || a.LS / 2 < points + ((points - 1) >> 3))
+            return hipErrorInvalidConfiguration;
+    }
     // the register-exchange kernels address contiguous lines (element stride 1)
     if (fixed && fixed->table == FT_WAVE1024 && (a.in_es != 1 || a.out_es != 1 || !a.tw))
         return hipErrorInvalidConfiguration;

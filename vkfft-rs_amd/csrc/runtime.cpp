@@ -15,6 +15,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <numeric>
 #include <sstream>
 #include <string>
 #include <vector>
@@ -1454,6 +1455,108 @@ bool shares_lines(size_t inner, int G, int prec) {
 
 // Axes whose bit is set in `omit` are left untransformed (the real axis of an
 // N-D real transform).
+// Stage radices of a field's axis: the fewest stages, and of those the smallest
+// sum of radices (stages cost a pass over LDS and a barrier each). wide: with
+// radices 12 and 16.
+bool field_schedule(int n, bool wide, int top, std::vector<int>& cur, std::vector<int>& best) {
+    if (n == 1) {
+        auto sum = [](const std::vector<int>& v) { return std::accumulate(v.begin(), v.end(), 0); };
+        if (best.empty() || cur.size() < best.size() || (cur.size() == best.size() && sum(cur) < sum(best))) best = cur;
+        return true;
+    }
+    bool any = false;
+    for (int r : {16, 13, 12, 11, 10, 9, 8, 7, 6, 5, 4, 3, 2}) {
+        if (r > top || n % r || (!wide && r >= 12 && r != 13) || (!best.empty() && cur.size() >= best.size())) continue;
+        cur.push_back(r);
+        any |= field_schedule(n / r, wide, r, cur, best);
+        cur.pop_back();
+    }
+    return any;
+}
+
+// Small fields in one kernel (KK_FIELD) where both LDS buffers of a field fit a
+// CU. Returns false where the axis passes below are kept; us, axis passes against
+// one kernel, for 2-D fields:
+// - power-of-two axes of 16 and more whose field takes the CU to itself (above
+//   80 KB): f64 64 x 64 7.2 against 8.6, x 1025 46.9 against 55.0;
+// - such fields with radices above 10 beyond two rounds of blocks: f32 91 x 77 x
+//   1141 77.4 against 90.5 (x 142: 23.2 against 15.9, one kernel);
+// - f32 fields of 1024 points and more with other factors, both axes on fixed
+//   shapes, above 48 MB (the passes stream at the Infinity Cache's rate): 60 x 60 x
+//   2222 64.3 against 65.9, 48 x 96 x 1736 64.1 against 66.7; at 8 MB 18.7 against 14.2
+//   and 22.8 against 10.9. f64 gains there too (60 x 60 x 1166 65.4 against 57.8).
+bool plan_field(Ctx& c, const vkfx_plan_desc& d, int* rc) {
+    *rc = VKFX_OK;
+    // VKFX_FIELD=0 keeps the axis passes (comparison runs), as does the request for
+    // a shape of theirs
+    if (const char* e = getenv("VKFX_FIELD"); e && e[0] == '0') return false;
+    if (const char* e = getenv("VKFX_REGISTER_EXCHANGE"); e && e[0] == '1') return false;
+    if (d.rank < 2 || d.rank > 3) return false;
+    const int prec = c.prec;
+    const size_t cs = csize(prec);
+    size_t total = 1;
+    bool pow2 = true, fixed = true, short_axis = false;
+    for (uint32_t i = 0; i < d.rank; ++i) {
+        const size_t n = d.dims[i];
+        if (d.axis_algorithm[i] != VKFX_ALG_STOCKHAM || n < 2 || n > 8192) return false;
+        total *= n;
+        if (total > 16384) return false;
+        pow2 &= (n & (n - 1)) == 0;
+        short_axis |= n < 16;
+        fixed &= find_fixed(KK_PLAIN, prec, d.direction, (int)n, i + 1 < d.rank) != nullptr;
+    }
+    auto buffers = [&](size_t points) { return 2 * ((points + (points >> 3) + 2) / 2 * 2); };
+    if (buffers(total) * cs > std::min<size_t>(c.lds_max, 156 * 1024)) return false;
+    const bool alone = buffers(total) * cs > 80 * 1024;
+    KArgs a = blank();
+    std::vector<int> radix;
+    for (int ax = 0; ax < 3; ++ax) {
+        field_dim(a, ax) = 1;
+        if (ax >= (int)d.rank) continue;
+        const size_t n = d.dims[d.rank - 1 - ax];
+        std::vector<int> r, cur;
+        // the f64 radix 16 (212 registers) where the LDS leaves one block per CU
+        // anyway: 16^3 x 1025 73.0 -> 59.6
+        if (!field_schedule((int)n, !prec || (alone && pow2), 16, cur, r)) return false;
+        field_dim(a, ax) = (int)n;
+        field_stages(a, ax) = (int)r.size();
+        radix.insert(radix.end(), r.begin(), r.end());
+    }
+    if (radix.size() > (size_t)kMaxStages) return false;
+    if (d.rank == 2) {
+        if (alone && pow2 && !short_axis) return false;
+        if (alone && d.batch > 512 && *std::max_element(radix.begin(), radix.end()) > 10) return false;
+        if (!prec && !pow2 && fixed && total >= 1024 && total * d.batch * cs > (48u << 20)) return false;
+    }
+    // fields packed into a block while at least 512 blocks remain: up to 4096 f32 or
+    // 1024 f64 points (f64 30 x 14 x 2380 15.7 against 21.7 with 2048 points; f32 within
+    // 2% from 1024 to 4096)
+    const size_t fill = (prec ? 1024 : 4096) / total;
+    field_pack(a) = (int)std::max<size_t>(1, std::min<size_t>(fill, d.batch / 512));
+    const size_t points = total * field_pack(a);
+    // a direct first stage reads runs of n / R elements; shorter runs than 64 bytes are copied in
+    if ((size_t)(field_dim(a, 0) / radix[0]) * cs < 64) a.flags |= KF_FIELD_COPY;
+    a.N = (int)total;
+    a.G = 1;
+    a.TT = (int)std::min<size_t>(512, std::max<size_t>(64, (points / 8 + 63) / 64 * 64));
+    a.LS = (int)buffers(points);
+    a.nstages = (int)radix.size();
+    for (int i = 0; i < a.nstages; ++i) {
+        a.radix[i] = radix[i];
+        if (radix[i] > 10) a.flags |= KF_FIELD_LARGE;
+    }
+    a.nlines = (long long)d.batch;
+    a.in_es = a.out_es = 1;
+    a.in_os = a.out_os = (long long)total;
+    if (d.direction > 0 && d.normalize) a.scale = 1.0 / (double)total;
+    for (int ax = 0; ax < (int)d.rank; ++ax)
+        if ((*rc = stage_table(c.p, (size_t)field_dim(a, ax), prec, &field_roots(a, ax)))) return true;
+    Launch L{KK_FIELD, d.direction, a, blocks_for((long long)d.batch, field_pack(a)), (unsigned)a.TT, (size_t)a.LS * cs,
+             SEL_IN, SEL_OUT, 0, 0, "field", nullptr, c.cur_chunk};
+    c.p->launches.push_back(L);
+    return true;
+}
+
 int plan_c2c_nd(Ctx& c, const vkfx_plan_desc& d, uint32_t omit) {
     const int prec = c.prec;
     const int dir = d.direction;
@@ -2683,6 +2786,11 @@ int vkfx_plan_create(vkfx_context* ctx, const vkfx_plan_desc* desc_in, vkfx_plan
             return rc;
         }
     }
+    // dense tensors of the compute type with no zero intervals and the device's own tuning
+    bool plain_tensor = (d.precision == VKFX_F32 || d.precision == VKFX_F64) && !d.custom_tuning && !d.in_batch_stride &&
+                        !d.out_batch_stride;
+    for (uint32_t i = 0; i < d.rank; ++i)
+        plain_tensor = plain_tensor && !d.in_axis_stride[i] && !d.out_axis_stride[i] && !d.zero_left[i] && !d.zero_right[i];
     try {
         if (conv_real) {
             p->in_bytes = conv_coords * total * rs;
@@ -2704,7 +2812,7 @@ int vkfx_plan_create(vkfx_context* ctx, const vkfx_plan_desc* desc_in, vkfx_plan
                 size_t conv = d.convolution_len[0];
                 if (alg == VKFX_ALG_RADER) conv = 0;  // Bluestein fallback uses M = next smooth >= 2N-1
                 rc = plan_c2c_1d(c, d.dims[0], d.batch, d.direction, d.normalize != 0, a, conv);
-            } else {
+            } else if (!plain_tensor || d.omit_dimension || !plan_field(c, d, &rc)) {
                 rc = plan_c2c_nd(c, d, d.omit_dimension);
             }
         } else if (r2r) {
