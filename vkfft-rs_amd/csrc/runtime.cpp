@@ -842,7 +842,12 @@ void note_pass(Ctx& c, const Launch& L) {
          << ",\"pair_loads\":" << ((L.a.flags & KF_PAIR_LOADS) ? "true" : "false")
          << ",\"radices\":[";
     for (int i = 0; i < L.a.nstages; ++i) c.js << (i ? "," : "") << L.a.radix[i];
-    c.js << "]}";
+    c.js << "]";
+    // a field's axes, last one first: how many of the radices are each axis's
+    if (L.kind == KK_FIELD)
+        c.js << ",\"axis_stages\":[" << field_stages(L.a, 0) << "," << field_stages(L.a, 1) << "," << field_stages(L.a, 2)
+             << "],\"fields_per_block\":" << field_pack(L.a);
+    c.js << "}";
 }
 
 // Launches whose blocks share HBM cache lines with their neighbours get their
@@ -1474,6 +1479,23 @@ bool field_schedule(int n, bool wide, int top, std::vector<int>& cur, std::vecto
     return any;
 }
 
+// VKFX_FIELD=0 keeps the axis passes (comparison runs), VKFX_FIELD=1 takes fields
+// wherever plan_field's rule does. Unset, a knob that selects the axis passes'
+// kernels or LDS budget keeps them, and the index-map test build does too: its
+// pass list names the passes whose addresses it checks.
+bool field_wanted() {
+    if (const char* e = getenv("VKFX_FIELD")) return e[0] != '0';
+#ifdef VKFX_INDEX_TEST
+    return false;
+#else
+    auto set = [](const char* name) {
+        const char* e = getenv(name);
+        return e && e[0] == '1';
+    };
+    return !set("VKFX_REGISTER_EXCHANGE") && !set("VKFX_DISABLE_FIXED") && !getenv("VKFX_LDS_BUDGET_KB");
+#endif
+}
+
 // Small fields in one kernel (KK_FIELD) where both LDS buffers of a field fit a
 // CU. Returns false where the axis passes below are kept; us, axis passes against
 // one kernel, for 2-D fields:
@@ -1487,10 +1509,7 @@ bool field_schedule(int n, bool wide, int top, std::vector<int>& cur, std::vecto
 //   and 22.8 against 10.9. f64 gains there too (60 x 60 x 1166 65.4 against 57.8).
 bool plan_field(Ctx& c, const vkfx_plan_desc& d, int* rc) {
     *rc = VKFX_OK;
-    // VKFX_FIELD=0 keeps the axis passes (comparison runs), as does the request for
-    // a shape of theirs
-    if (const char* e = getenv("VKFX_FIELD"); e && e[0] == '0') return false;
-    if (const char* e = getenv("VKFX_REGISTER_EXCHANGE"); e && e[0] == '1') return false;
+    if (!field_wanted()) return false;
     if (d.rank < 2 || d.rank > 3) return false;
     const int prec = c.prec;
     const size_t cs = csize(prec);
