@@ -848,6 +848,15 @@ def b(v):
     return "true" if v else "false"
 
 
+# Tables whose shapes read every twiddle of a stage from a per-stage table: radices
+# of 9 to 12 as products of one root lost precision against the two passes of a
+# split axis (f32 columns of 1000 over rows of 42: 1.89e-7 split, 2.74e-7 as products,
+# 1.70e-7 from tables; 1080 x 1920 3.14e-7, 3.28e-7, 2.81e-7; f64 960 x 540 6.4e-16,
+# 7.0e-16, 6.2e-16), at the same times (1080 x 1920 x 4 58.7 us as products, 58.4 from
+# tables, 1024 x 1024 x 8 56.9 and 56.7; convolutions of one 1024 x 1024 f32 31.8 and 32.7).
+STAGE_TABLES = ("kf_cols_f32", "kf_cols_f64")
+
+
 def render(name):
     """Text of table file `name`.hip."""
     prec = 1 if name.endswith("f64") else 0
@@ -863,7 +872,8 @@ def render(name):
             continue
         kind, io, N, TT, G, col, rad, PS, LS = it
         for S, nti, nto in roles(kind, col):
-            lines.append(f"    VKFX_SHAPE(KK_{kind}, Io{io}, {T}, {prec}, {S}, {N}, {TT}, {G}, {PS}, {LS}, {b(col)}, "
+            macro = "VKFX_FIXED_T" if name in STAGE_TABLES else "VKFX_SHAPE"
+            lines.append(f"    {macro}(KK_{kind}, Io{io}, {T}, {prec}, {S}, {N}, {TT}, {G}, {PS}, {LS}, {b(col)}, "
                          f"{b(nti)}, {b(nto)}, {', '.join(map(str, rad))}),")
     lines += ["};", "", f"const FixedKernel* {FUNCS[name]}(int* count) {{",
               "    *count = (int)(sizeof(kTable) / sizeof(kTable[0]));", "    return kTable;", "}", "",
