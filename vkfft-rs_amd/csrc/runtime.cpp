@@ -22,6 +22,7 @@
 
 #include "kernels.hpp"
 #include "planner.hpp"
+#include "roots.hpp"
 #include "vkfx.h"
 
 using namespace vkfx;
@@ -51,14 +52,7 @@ struct DevBuf {
 };
 
 typedef long double ld;
-const ld kPi = 3.141592653589793238462643383279502884L;
-
-// exp(-2 pi i k / n) with exact integer reduction of k.
-void root(ld k, ld n, ld& c, ld& s) {
-    ld a = -2.0L * kPi * k / n;
-    c = cosl(a);
-    s = sinl(a);
-}
+const ld kPi = kPiL;
 
 }  // namespace
 
@@ -429,8 +423,8 @@ int stage_table(vkfx_plan* p, size_t n, int prec, const void** dev) {
         *dev = p->table_cache[key];
         return VKFX_OK;
     }
-    std::vector<ld> re(n), im(n);
-    for (size_t k = 0; k < n; ++k) root((ld)k, (ld)n, re[k], im[k]);
+    std::vector<ld> re, im;
+    roots(n, re, im);
     auto b = pack(re, im, prec);
     return upload(p, key, b.data(), b.size(), dev);
 }
@@ -461,17 +455,17 @@ int stage_pr_table(vkfx_plan* p, const FixedKernel* f, int prec, const void** de
         *dev = p->table_cache[key];
         return VKFX_OK;
     }
-    std::vector<ld> re, im;
+    std::vector<ld> re, im, wr, wi;
+    roots((size_t)f->N, wr, wi);
     long long P = 1;
     for (int s = 0; s < f->nst; ++s) {
-        const long long R = f->radix[s];
+        const long long R = f->radix[s], step = f->N / (P * R);
         if (P > 1)
             for (long long k = 0; k < P; ++k)
                 for (long long i = 1; i < R; ++i) {
-                    ld x, y;
-                    root((ld)((k * i) % (P * R)), (ld)(P * R), x, y);
-                    re.push_back(x);
-                    im.push_back(y);
+                    const size_t at = (size_t)((k * i) % (P * R) * step);
+                    re.push_back(wr[at]);
+                    im.push_back(wi[at]);
                 }
         P *= R;
     }
@@ -585,25 +579,28 @@ int rader_stage_tables(vkfx_plan* p, const std::vector<int>& radix, int prec, KA
 }
 
 // Two-level table for exp(-2 pi i k/L), k <= L: lo[j] = root(j), j < 2^s;
-// hi[h] = root(h*2^s). The kernels form hi[k>>s]*lo[k&(2^s-1)].
+// hi[h] = root(h*2^s). The kernels form hi[k>>s]*lo[k&(2^s-1)]. Both levels are one
+// allocation and one copy (about 10 us of a plan's creation each).
 int two_level(vkfx_plan* p, size_t L, int prec, const void** lo, const void** hi, int* shift) {
     int s = 0;
     while (((size_t)1 << (2 * s)) < L + 1) ++s;
     s = std::max(s, 1);
     const size_t nlo = (size_t)1 << s, nhi = (L >> s) + 2;
-    std::string key = "tl:" + std::to_string(L) + ":" + std::to_string(prec);
-    std::vector<ld> re(nlo), im(nlo);
-    for (size_t j = 0; j < nlo; ++j) root((ld)j, (ld)L, re[j], im[j]);
-    auto b = pack(re, im, prec);
-    int rc = upload(p, key + ":lo", b.data(), b.size(), lo);
-    if (rc) return rc;
-    re.assign(nhi, 0);
-    im.assign(nhi, 0);
-    for (size_t h = 0; h < nhi; ++h) root((ld)(h << s), (ld)L, re[h], im[h]);
-    b = pack(re, im, prec);
-    rc = upload(p, key + ":hi", b.data(), b.size(), hi);
+    const std::string key = "tl:" + std::to_string(L) + ":" + std::to_string(prec);
     *shift = s;
-    return rc;
+    auto it = p->table_cache.find(key);
+    if (it != p->table_cache.end()) {
+        *lo = it->second;
+    } else {
+        std::vector<ld> re(nlo + nhi), im(nlo + nhi);
+        for (size_t j = 0; j < nlo; ++j) root((ld)j, (ld)L, re[j], im[j]);
+        for (size_t h = 0; h < nhi; ++h) root((ld)(h << s), (ld)L, re[nlo + h], im[nlo + h]);
+        auto b = pack(re, im, prec);
+        int rc = upload(p, key, b.data(), b.size(), lo);
+        if (rc) return rc;
+    }
+    *hi = (const char*)*lo + nlo * (prec ? 16 : 8);
+    return VKFX_OK;
 }
 
 // Bluestein chirp c[n] = exp(sign * pi i n^2 / N) with n^2 reduced mod 2N
