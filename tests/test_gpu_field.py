@@ -44,6 +44,38 @@ def test_fields(hip_ctx, monkeypatch, dims, batch, one32, one64, prec):
     assert all(p["kernel"] != "field" for p in other.describe()["passes"])
 
 
+# fields alone on a CU: (dims, batch, precision, one kernel by the rule of 256 CUs)
+ALONE = [([20, 20, 20], 1, "f32", False), ([16, 16, 16], 1, "f64", True), ([12, 12, 20], 1, "f64", False),
+         ([8, 30, 36], 255, "f32", False), ([8, 30, 36], 256, "f32", True), ([18, 18, 18], 256, "f32", False),
+         ([25, 320], 1, "f32", False), ([36, 225], 1, "f32", False), ([15, 540], 300, "f32", False),
+         ([8, 512], 1, "f64", False), ([8, 512], 15, "f64", True), ([8, 512], 16, "f64", False), ([8, 512], 256, "f64", True), ([45, 64], 1, "f64", False),
+         ([48, 108], 1, "f32", True), ([100, 80], 1, "f32", True), ([160, 50], 1, "f32", False), ([160, 50], 256, "f32", True),
+         ([1000, 8], 1, "f32", False), ([270, 30], 256, "f32", False), ([80, 60], 513, "f32", False), ([91, 77], 57, "f32", True),
+         ([4, 2000], 31, "f32", False), ([4, 2000], 32, "f32", True), ([9, 792], 1, "f32", False), ([1024, 4], 1, "f64", True), ([2, 2, 1000], 1, "f64", True)]
+
+
+@pytest.mark.parametrize("dims,batch,prec,one", ALONE)
+def test_alone_on_a_cu(hip_ctx, monkeypatch, dims, batch, prec, one):
+    """Both sides of the rule for fields whose LDS takes the CU, and the same
+    results from the one kernel where the rule keeps the axis passes."""
+    if hip_ctx.device_profile()["compute_units"] != 256:
+        pytest.skip("the rule's sides are stated for 256 CUs")
+    wide = prec == "f64"
+    x = o.complex_uniform(int(np.prod(dims)) * batch, 5, np.complex128 if wide else np.complex64)
+    axes = tuple(range(1, len(dims) + 1))
+    ref = np.fft.fftn(x.astype(np.complex128).reshape([batch] + dims), axes=axes).reshape(-1)
+    for env in (None, "1"):
+        if env:
+            monkeypatch.setenv("VKFX_FIELD", env)
+        ctx = vk.HipExecutionContext(0)
+        try:
+            ir = _plan(ctx, dims, batch, vk.Precision.F64 if wide else vk.Precision.F32, vk.Direction.Forward)
+            assert o.rel_l2(ctx.execute_transform(ir, x), ref) <= (4e-15 if wide else 1e-6)
+            assert ([p["kernel"] for p in ctx.plan(ir).describe()["passes"]] == ["field"]) == (one or env == "1")
+        finally:
+            ctx.close()
+
+
 @pytest.mark.parametrize("dims,batch", [([64, 64], 2), ([30, 14], 1100), ([8, 9, 10], 7)])
 def test_in_place(hip_ctx, dims, batch):
     import torch

@@ -1476,42 +1476,77 @@ bool field_schedule(int n, bool wide, int top, std::vector<int>& cur, std::vecto
     return any;
 }
 
-// VKFX_FIELD=0 keeps the axis passes (comparison runs), VKFX_FIELD=1 takes fields
-// wherever plan_field's rule does. Unset, a knob that selects the axis passes'
-// kernels or LDS budget keeps them, and the index-map test build does too: its
-// pass list names the passes whose addresses it checks.
-bool field_wanted() {
-    if (const char* e = getenv("VKFX_FIELD")) return e[0] != '0';
+// VKFX_FIELD=0 keeps the axis passes (comparison runs), VKFX_FIELD=1 takes every
+// field that fits (tests). Unset, plan_field's rule decides, a knob that selects the
+// axis passes' kernels or LDS budget keeps them, and the index-map test build does
+// too: its pass list names the passes whose addresses it checks.
+enum FieldWanted { FIELD_OFF, FIELD_BY_RULE, FIELD_ALL };
+FieldWanted field_wanted() {
+    if (const char* e = getenv("VKFX_FIELD")) return e[0] == '0' ? FIELD_OFF : FIELD_ALL;
 #ifdef VKFX_INDEX_TEST
-    return false;
+    return FIELD_OFF;
 #else
     auto set = [](const char* name) {
         const char* e = getenv(name);
         return e && e[0] == '1';
     };
-    return !set("VKFX_REGISTER_EXCHANGE") && !set("VKFX_DISABLE_FIXED") && !getenv("VKFX_LDS_BUDGET_KB");
+    const bool off = set("VKFX_REGISTER_EXCHANGE") || set("VKFX_DISABLE_FIXED") || getenv("VKFX_LDS_BUDGET_KB");
+    return off ? FIELD_OFF : FIELD_BY_RULE;
 #endif
 }
 
 // Small fields in one kernel (KK_FIELD) where both LDS buffers of a field fit a
 // CU. Returns false where the axis passes below are kept; us, axis passes against
-// one kernel, for 2-D fields:
-// - power-of-two axes of 16 and more whose field takes the CU to itself (above
-//   80 KB): f64 64 x 64 7.2 against 8.6, x 1025 46.9 against 55.0;
-// - such fields with radices above 10 beyond two rounds of blocks: f32 91 x 77 x
-//   1141 77.4 against 90.5 (x 142: 23.2 against 15.9, one kernel);
-// - f32 fields of 1024 points and more with other factors, both axes on fixed
+// one kernel:
+// - 2-D fields of power-of-two axes of 16 and more that take the CU to themselves
+//   (above 80 KB): f64 64 x 64 7.2 against 8.6, x 1025 46.9 against 55.0;
+// - 2-D fields alone on a CU beyond two rounds of blocks, with radices above 10 or
+//   in f32: 91 x 77 x 1141 77.4 against 90.5 (x 142: 23.2 against 15.9, one kernel),
+//   80 x 60 x 625 31.6 against 33.5; f64 64 x 48 x 1302 73.0 against 53.5;
+// - other fields alone on a CU where the kernel's stages are long against the passes
+//   (field_slow);
+// - f32 2-D fields of 1024 points and more with other factors, both axes on fixed
 //   shapes, above 48 MB (the passes stream at the Infinity Cache's rate): 60 x 60 x
 //   2222 64.3 against 65.9, 48 x 96 x 1736 64.1 against 66.7; at 8 MB 18.7 against 14.2
 //   and 22.8 against 10.9. f64 gains there too (60 x 60 x 1166 65.4 against 57.8).
+//
+// field_slow, for fields alone on a CU: `trips` is the sum over the stages of the
+// butterflies a thread runs one after another (about 0.7 us each beside 5 us);
+// `quick`: every strided axis is on a fixed shape or on a runtime shape nearly as
+// fast (12 points and more without the factors 7, 11 and 13). us, axis passes
+// against one kernel:
+// - fewer blocks than CUs, 3-D: 20^3 11.5 against 17.5 (24 trips), 30 x 30 x 9 13.1
+//   against 15.6 (16), f64 12 x 12 x 20 11.2 against 12.3 (14), 16^3 14.3 against 8.5 (3);
+// - 2-D over columns below 48 points, whose two passes take 7 to 9: 25 x 320 7.8 against
+//   13.4, 9 x 792 8.5 against 11.8, 36 x 240 7.6 against 14.3, f64 45 x 64 7.8 against
+//   8.9; 8 x 512 f64 (4 trips) 7.1 against 8.9, x 2 8.4 against 9.1, x 50 8.9 against 9.9,
+//   x 384 25.5 against 21.6;
+// - 2-D over longer columns (10 to 13): 48 x 108 12.8 against 10.0 (7 trips), 100 x 80
+//   13.7 against 11.9 (8), 81 x 64 9.8 against 10.0 (8), 128 x 65 8.9 against 14.3 (15), 160 x 50 11.8 against 13.3 (9),
+//   270 x 30 11.6 against 16.2 (16); short rows 1000 x 8 12.8 against 13.8 (8);
+// - every CU at work: 3-D 8 x 30 x 36 x 347 39.7 against 35.7 (16 trips), 18^3 x 514 42.7
+//   against 49.8 (18); 2-D 72 x 120 x 347 33.1 against 26.7 (9), 300 x 12 x 416 f64 31.3
+//   against 27.4 (10), 200 x 40 x 384 32.9 against 34.9 (16);
+// - short axes without a fixed shape, 2-D: 4 x 2000 13.1 against 13.8 (16 trips), x 50 19.7
+//   against 14.6; 2 x 2048 f64 9.3 against 9.8 (7), x 50 32.4
+//   against 10.5; 1024 x 4 f64 11.4 against 10.1 (5).
+bool field_slow(const vkfx_plan_desc& d, int trips, bool quick, bool smooth, size_t cus) {
+    const bool full = d.batch >= cus;
+    if (!quick) return d.rank == 2 && smooth && d.batch < 32 && trips >= 7;
+    if (d.rank == 3) return trips > (full ? 16 : 7);
+    if (d.dims[0] < 48) return trips > 4 || d.batch < 2 || (d.batch >= 16 && !full);
+    return trips > (full ? 11 : d.dims[1] < 16 ? 7 : 8);
+}
+
 bool plan_field(Ctx& c, const vkfx_plan_desc& d, int* rc) {
     *rc = VKFX_OK;
-    if (!field_wanted()) return false;
+    const FieldWanted wanted = field_wanted();
+    if (wanted == FIELD_OFF) return false;
     if (d.rank < 2 || d.rank > 3) return false;
     const int prec = c.prec;
     const size_t cs = csize(prec);
     size_t total = 1;
-    bool pow2 = true, fixed = true, short_axis = false;
+    bool pow2 = true, fixed = true, smooth = true, quick = true, short_axis = false;
     for (uint32_t i = 0; i < d.rank; ++i) {
         const size_t n = d.dims[i];
         if (d.axis_algorithm[i] != VKFX_ALG_STOCKHAM || n < 2 || n > 8192) return false;
@@ -1519,7 +1554,11 @@ bool plan_field(Ctx& c, const vkfx_plan_desc& d, int* rc) {
         if (total > 16384) return false;
         pow2 &= (n & (n - 1)) == 0;
         short_axis |= n < 16;
-        fixed &= find_fixed(KK_PLAIN, prec, d.direction, (int)n, i + 1 < d.rank) != nullptr;
+        const bool last = i + 1 == d.rank, has = find_fixed(KK_PLAIN, prec, d.direction, (int)n, !last) != nullptr;
+        const bool five = n % 7 && n % 11 && n % 13;
+        fixed &= has;
+        smooth &= five;
+        quick &= has || last || (five && n >= 12);
     }
     auto buffers = [&](size_t points) { return 2 * ((points + (points >> 3) + 2) / 2 * 2); };
     if (buffers(total) * cs > std::min<size_t>(c.lds_max, 156 * 1024)) return false;
@@ -1539,9 +1578,16 @@ bool plan_field(Ctx& c, const vkfx_plan_desc& d, int* rc) {
         radix.insert(radix.end(), r.begin(), r.end());
     }
     if (radix.size() > (size_t)kMaxStages) return false;
-    if (d.rank == 2) {
+    auto threads = [](size_t n) { return (int)std::min<size_t>(512, std::max<size_t>(64, (n / 8 + 63) / 64 * 64)); };
+    if (alone && wanted == FIELD_BY_RULE) {
+        int trips = 0;
+        for (int r : radix) trips += ((int)total / r + threads(total) - 1) / threads(total);
+        const size_t cus = c.p->ctx->profile.compute_units;
+        if (field_slow(d, trips, quick, smooth, cus ? cus : 256)) return false;
+    }
+    if (d.rank == 2 && wanted == FIELD_BY_RULE) {
         if (alone && pow2 && !short_axis) return false;
-        if (alone && d.batch > 512 && *std::max_element(radix.begin(), radix.end()) > 10) return false;
+        if (alone && d.batch > 512 && ((!prec && quick) || *std::max_element(radix.begin(), radix.end()) > 10)) return false;
         if (!prec && !pow2 && fixed && total >= 1024 && total * d.batch * cs > (48u << 20)) return false;
     }
     // fields packed into a block while at least 512 blocks remain: up to 4096 f32 or
@@ -1554,7 +1600,7 @@ bool plan_field(Ctx& c, const vkfx_plan_desc& d, int* rc) {
     if ((size_t)(field_dim(a, 0) / radix[0]) * cs < 64) a.flags |= KF_FIELD_COPY;
     a.N = (int)total;
     a.G = 1;
-    a.TT = (int)std::min<size_t>(512, std::max<size_t>(64, (points / 8 + 63) / 64 * 64));
+    a.TT = threads(points);
     a.LS = (int)buffers(points);
     a.nstages = (int)radix.size();
     for (int i = 0; i < a.nstages; ++i) {
