@@ -80,6 +80,22 @@ def test_convolution(hip_ctx, n, inner, batch, prec):
     assert o.rel_l2(y, ref) <= (2e-13 if wide else 2e-6)
 
 
+@pytest.mark.parametrize("n,inner,fused", [(900, 16, True), (972, 16, False), (1080, 112, False), (1080, 120, True),
+                                           (1125, 360, False), (1125, 375, True), (1215, 49, False), (1024, 16, True),
+                                           (832, 16, True)])
+def test_convolution_of_few_columns(hip_ctx, n, inner, fused):
+    """Axes that the plain plan splits: one fused kernel per column, or the split
+    passes around the multiply where few blocks would leave the CUs idle."""
+    x, k = o.complex_uniform(n * inner, 7, np.complex64), o.complex_uniform(n * inner, 8, np.complex64)
+    conv = vk.ConvolutionIr.build(vk.FftConfig.new([n, inner]), k)
+    y = hip_ctx.execute_convolution(conv, x)
+    ref = np.fft.ifft2(np.fft.fft2(x.astype(np.complex128).reshape(n, inner)) * k.astype(np.complex128).reshape(n, inner))
+    assert o.rel_l2(y, ref.reshape(-1)) <= 2e-6
+    plan = vk.Plan(hip_ctx, conv.ir, desc=conv.desc())
+    names = [p["kernel"] for p in plan.describe()["passes"]]
+    assert ("convolution_fused_axis0" in names) == fused and ("convolution_multiply" in names) != fused, names
+
+
 @pytest.mark.parametrize("prec,tol", [(vk.Precision.F16StorageF32Compute, 1e-3),
                                       (vk.Precision.F64ComputeF32Storage, 1e-7)])
 def test_mixed_storage(hip_ctx, prec, tol):

@@ -2141,12 +2141,18 @@ int plan_convolution(Ctx& c, const vkfx_plan_desc& d, size_t coords, size_t out_
     // data instead of 2D + 1 (the multiply folded into the last forward /
     // first inverse axis, as the reference folds it into its uploads), or
     // 2D - 1 instead of 2D + 3 where the plain plan splits axis 0 into two
-    // passes per direction. Taken with a fixed-shape column kernel for N0, or
-    // where axis 0 would be split (its runtime-shape column kernel then still
-    // wins); an axis 0 of one pass without a fixed-shape kernel keeps the
-    // separate multiply, since its fixed-shape FFT column passes beat the
-    // runtime-shape fused kernel ([128, 128, 128] x 4 f32 before the fixed
-    // column kernel: 192 us unfused, 201 us fused).
+    // passes per direction. An axis 0 of one pass takes it with a fixed-shape
+    // column kernel for N0; without one it keeps the separate multiply, since its
+    // fixed-shape FFT column passes beat the runtime-shape fused kernel ([128, 128,
+    // 128] x 4 f32 before the fixed column kernel: 192 us unfused, 201 us fused).
+    // An axis 0 that would be split takes it in f32 on the runtime shape (four
+    // passes saved; f64 lines of those lengths leave fewer than 8 columns a block)
+    // and, up to 1247 points, on the fixed shape in place of that (1024 x 48 50 against
+    // 39.5) or where its blocks, one a CU, are short or many enough against the split
+    // passes, which spread a line over the CUs. Measured, us, separate against fused: 900 points, 3 blocks 39.5 against 38.9;
+    // 972 3 blocks 39.0 against 40.3, 9 blocks 37.0 against 36.4; 1080 39.2 against 41.3,
+    // 37.5 against 36.7; 1125 9 blocks 37.8 against 40.8, 24 blocks 41.8 against 39.6; 1215
+    // 13 blocks 34.2 against 40.0, 24 blocks 43.8 against 43.1, 96 blocks 64.4 against 49.0.
     size_t sl1 = 0, sl2 = 0;
     bool nd_fused = d.rank >= 2 && !ca.matrix && ca.kernel_count <= 1 && coords == 1 && d.dims[0] > 1;
     for (uint32_t i = 0; nd_fused && i < d.rank; ++i) nd_fused = d.axis_algorithm[i] == VKFX_ALG_STOCKHAM;
@@ -2154,11 +2160,12 @@ int plan_convolution(Ctx& c, const vkfx_plan_desc& d, size_t coords, size_t out_
         const size_t n0 = d.dims[0], rest = T / n0;
         const bool split = split_strided_axis(c, n0, d.batch * rest, &sl1, &sl2);
         Geometry g = kernel_geometry(KK_CONV_1, c.prec, -1, n0, true, c.prec ? 8 : 16, c.lds_max, c.lds_budget);
+        const size_t blocks = g.ok ? (d.batch * rest + g.G - 1) / g.G : 0;
+        const bool fills = n0 <= 900 || blocks >= (n0 <= 1080 ? 8 : 24) ||
+                           geometry(n0, c.prec, 16, c.lds_max, c.lds_budget).G >= 8;
         // strided columns: at least 8 adjacent columns per block, so each
         // HBM access moves 64 bytes or more
-        // and in f64 only where the plain plan takes one pass (a split axis has
-        // too few lines to fill the CUs with whole columns)
-        if (g.ok && g.G >= 8 && (split ? !c.prec : g.fixed != nullptr)) {
+        if (g.ok && g.G >= 8 && (split ? !c.prec && fills : g.fixed != nullptr)) {
             c.js << ",\"fused\":true,\"fused_axis\":0},";
             int rc = transform(d.batch, -1, false, SEL_IN, SEL_FULL, 1u);
             if (rc) return rc;
