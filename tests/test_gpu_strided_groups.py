@@ -33,3 +33,20 @@ def test_strided_passes(hip_ctx, dims, batch, prec):
         assert p["xcd_groups"] == shared, p
         if shared and p["fixed_shape"]:
             assert p["nontemporal"] == [False, False], p
+
+
+@pytest.mark.parametrize("dims,batch,shared", [([24, 405], 6, True), ([24, 405], 7, False), ([24, 405], 539, False),
+                                               ([24, 405], 540, True), ([127, 405], 2, False), ([128, 405], 2, True),
+                                               ([24, 400], 540, False), ([200, 120], 4, False)])
+def test_rule_by_size(hip_ctx, dims, batch, shared):
+    """Short lines and pitches of half memory lines keep the round-robin order and nontemporal stores from 512 KB
+    to 40 MB, and everywhere where the row pitch is whole memory lines."""
+    x = o.complex_uniform(int(np.prod(dims)) * batch, 3, np.complex64)
+    ir = vk.TransformIr.build(vk.FftConfig.new(dims).with_batch_count(batch), vk.Direction.Forward)
+    y = hip_ctx.execute_transform(ir, x)
+    ref = np.fft.fft2(x.astype(np.complex128).reshape([batch] + dims)).reshape(-1)
+    assert o.rel_l2(y, ref) <= 2e-6
+    p = hip_ctx.plan(ir).describe()["passes"][-1]
+    assert p["xcd_groups"] == shared, p
+    if p["fixed_shape"]:
+        assert p["nontemporal"] == [False, not shared], p
