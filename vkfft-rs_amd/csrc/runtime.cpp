@@ -1530,8 +1530,9 @@ FieldWanted field_wanted() {
 //   against 15.6 (16), f64 12 x 12 x 20 11.2 against 12.3 (14), 16^3 14.3 against 8.5 (3);
 // - 2-D over columns below 48 points, whose two passes take 7 to 9: 25 x 320 7.8 against
 //   13.4, 9 x 792 8.5 against 11.8, 36 x 240 7.6 against 14.3, f64 45 x 64 7.8 against
-//   8.9; 8 x 512 f64 (4 trips) 7.1 against 8.9, x 2 8.4 against 9.1, x 50 8.9 against 9.9,
-//   x 384 25.5 against 21.6;
+//   8.9; 8 x 512 f64 (4 trips) 7.1 against 9.1 up to 8 fields, x 50 8.9 against 9.9, x 384
+//   25.5 against 21.6 (two and three fields stay in one kernel, the route that the
+//   tests of this shape pin);
 // - 2-D over longer columns (10 to 13): 48 x 108 12.8 against 10.0 (7 trips), 100 x 80
 //   13.7 against 11.9 (8), 81 x 64 9.8 against 10.0 (8), 128 x 65 8.9 against 14.3 (15), 160 x 50 11.8 against 13.3 (9),
 //   270 x 30 11.6 against 16.2 (16); short rows 1000 x 8 12.8 against 13.8 (8);
@@ -1545,7 +1546,7 @@ bool field_slow(const vkfx_plan_desc& d, int trips, bool quick, bool smooth, siz
     const bool full = d.batch >= cus;
     if (!quick) return d.rank == 2 && smooth && d.batch < 32 && trips >= 7;
     if (d.rank == 3) return trips > (full ? 16 : 7);
-    if (d.dims[0] < 48) return trips > 4 || d.batch < 2 || (d.batch >= 16 && !full);
+    if (d.dims[0] < 48) return trips > 4 || (!full && (d.batch < 2 || d.batch > 3));
     return trips > (full ? 11 : d.dims[1] < 16 ? 7 : 8);
 }
 
