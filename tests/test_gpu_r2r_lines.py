@@ -73,6 +73,35 @@ def test_strided_lines(hip_ctx, name, prec):
         _check(y, ref, n, prec)
 
 
+@pytest.mark.parametrize("name", KINDS)
+@pytest.mark.parametrize("prec", [vk.Precision.F32, vk.Precision.F64])
+def test_few_lines(hip_ctx, name, prec):
+    """Fewer blocks than CUs on the runtime shapes: lines spread over the CUs with
+    more threads than the stages need (at most the line's elements), along rows and
+    columns, and the three passes for lone strided lines that fill the LDS."""
+    import scipy.fft as sf
+    f = sf.dct if name.startswith("dct") else sf.dst
+    cus = hip_ctx.device_profile()["compute_units"]
+    dt = np.float32 if prec == vk.Precision.F32 else np.float64
+    for n, inner, batch in ((14, 1, 1), (28, 1, 3), (84, 1, cus), (84, 1, cus + 1), (154, 1, 3 * cus + 5), (1386, 1, 2),
+                            (4158, 1, 2), (14, 5, 3), (154, 30, 7), (1386, 9, 1), (2772, 33, 1)):
+        n += {"dct1": 1, "dst1": -1}.get(name, 0)
+        lines = batch * inner
+        x = o.uniform(n * lines, n + lines, dt)
+        ir = _plan(hip_ctx, name, [n, inner] if inner > 1 else [n], batch, prec, omit=(1,) if inner > 1 else ())
+        y = hip_ctx.execute_transform(ir, x)
+        _check(y, f(x.astype(np.float64).reshape(batch, n, inner), type=int(name[-1]), axis=1).reshape(-1), n, prec)
+        (p,) = hip_ctx.plan(ir).describe()["passes"]
+        assert p["kernel"] == "r2r_line", p
+        if not p["fixed_shape"] and lines < cus * 4:
+            G = p["lines_per_block"]
+            assert G <= -(-lines // cus) and p["block"] >= G * min(p["fft_len"], (512 if lines <= cus else 256) // G), p
+    n = {"dct1": 2049, "dst1": 2047, "dct4": 4096, "dst4": 4096}.get(name)
+    for inner, one in ((32, False), (33, True)) if n else ():
+        passes = hip_ctx.plan(_plan(hip_ctx, name, [n, inner], 1, prec, omit=(1,))).describe()["passes"]
+        assert (len(passes) == 1) == one, passes
+
+
 @pytest.mark.parametrize("name", ["dct2", "dct3", "dct4", "dct1", "dst2", "dst3"])
 def test_lines_stay_on_their_own(hip_ctx, name):
     """A line of NaN, of infinities or of tiny values leaves its neighbours

@@ -2310,13 +2310,42 @@ int plan_r2r(Ctx& c, size_t n, size_t batch, int kind, int dir, bool normalize, 
         const bool rows = inner == 1;
         const Geometry g0 = geometry(N, c.prec, 1, c.lds_max, c.lds_max);
         // strided lines: 32 (f32) / 16 (f64) adjacent lines, 128-byte segments
-        // of reals; rows: about 256 threads
+        // of reals, up to 64 of short ones to fill a wavefront (16 lines of one thread:
+        // f64 DCT-II 7 x 100000 and its rows 122 -> 131 us); rows: about 256 threads
         Geometry g = one_upload(N, c.prec, c.lds_max)
                          ? kernel_geometry(kind_r, c.prec, fft_dir, N, !rows,
-                                           rows ? std::max(1, 256 / g0.TT) : (c.prec ? 16 : 32), c.lds_max,
+                                           rows ? std::max(1, 256 / g0.TT)
+                                                : std::max(c.prec ? 16 : 32, std::min(64, 64 / g0.TT)), c.lds_max,
                                            rows ? c.lds_budget : c.lds_max)
                          : Geometry{};
-        if (g.ok) {
+        // Few lines on a runtime shape: spread over the CUs, with as many threads a
+        // line as its elements and 256 threads a block allow (512 with no more lines
+        // than CUs), whatever the stages need: a thread walks its share of the
+        // elements at both ends, each visit a chain of memory and table latencies.
+        // Measured, us, type and its inverse, pre pass / FFT / post pass against blocks
+        // sized for many lines and against this: f64 DST-IV 480 x 93 20.7, 31.7, 17; f64
+        // DST-I 59 x 1 21.1, 30.9, 11.8; f32 DCT-IV 28 x 600 37.9, 24.5, 11.6; f64 DST-II
+        // 84 x 3000 36.1, 31.8, 16.2; f32 DST-I 4095 x 1 23.6, 32.6, 24.0; columns f32 DCT-IV
+        // 96 x 500 88, 66, 28, f64 DCT-II 525 x 500 79, 88, 45.
+        if (g.ok && !g.fixed) {
+            const size_t units = p->ctx->profile.compute_units, cus = units ? units : 256;
+            if (batch < cus * (size_t)g.G) {
+                g.G = (int)((batch + cus - 1) / cus);
+                g.TT = std::max(g.TT, std::min(g.N, (batch <= cus ? 512 : 256) / g.G));
+                g.lds = (size_t)g.G * g.LS * csize(c.prec);
+            }
+        }
+        // A lone strided line reads a memory line an element, both extensions of type
+        // I twice and the ends of type IV against a half-length FFT in the three
+        // passes: up to 32 lines of 2048 points and more keep those, us, three passes
+        // against one kernel: f32 DST-I 8191 x 16 and its rows 84 against 106, 2047 x 16
+        // 46.3 against 49.4, DCT-I 3001 x 32 72.0 against 78.1, f64 DCT-IV 8192 x 16 55.8
+        // against 62.5; f64 DST-I 8191 x 64 128 against 90. The other forms where the rows
+        // are one memory line of f32: DCT-II 8192 x 32 57 against 66, 4096 x 32 46.7 against
+        // 50.5 (8192 x 16 64 against 53, x 64 79 against 58, f64 x 16 70 against 64).
+        const bool scattered = !rows && batch <= 32 && N >= 2048 &&
+                               (form == R2R_F_SYM || form == R2R_F_HALF || (!f64 && inner == 32));
+        if (g.ok && !scattered) {
             KArgs k = blank();
             k.C = (long long)inner;
             k.in_es = k.out_es = (long long)inner;
