@@ -25,6 +25,13 @@ int main() {
         // the axes and diagonals of the circle
         if (re[0] != 1.0L || im[0] != 0.0L) return std::printf("FAIL root 0 of %zu\n", n), 1;
         if (n % 2 == 0 && (re[n / 2] != -1.0L || im[n / 2] != 0.0L)) return std::printf("FAIL half of %zu\n", n), 1;
+        for (size_t count : {(size_t)0, (size_t)1, n / 4 + 1, n / 2, n - 1, n + 5}) {
+            std::vector<long double> a, b;
+            vkfx::roots(n, a, b, count);
+            if (a.size() != (count < n ? count : n)) return std::printf("FAIL count %zu of %zu\n", count, n), 1;
+            for (size_t k = 0; k < a.size(); ++k)
+                if (a[k] != re[k] || b[k] != im[k]) return std::printf("FAIL root %zu of %zu, first %zu\n", k, n, count), 1;
+        }
         if (n % 4 == 0 && (re[n / 4] != 0.0L || im[n / 4] != -1.0L)) return std::printf("FAIL quarter of %zu\n", n), 1;
     }
     std::printf("ok %zu\n", total);

@@ -364,11 +364,28 @@ __device__ __forceinline__ void root_powers(cpx<T> w, cpx<T>* p) {
     }
 }
 
+// p[i] = w^i, i < R, w = root `m` of a full table: the powers of two from the table,
+// the others as products of them, at most three factors each rounded once. A tree of
+// products from w alone (root_powers) squares w's own rounding error up to the
+// eighth power. For the kernels whose large radices would lose precision by it.
+template <int R, typename T>
+__device__ __forceinline__ void table_powers(const void* tw, int m, cpx<T>* p) {
+#pragma unroll
+    for (int i = 1; i < R; i *= 2) p[i] = ld_table<T>(tw, i * m);
+#pragma unroll
+    for (int i = 3; i < R; ++i) {
+        int hb = 1;
+        while (hb * 2 <= i) hb *= 2;
+        if (hb != i) p[i] = cmul(p[i - hb], p[hb]);
+    }
+}
+
 // Where a runtime-shape stage reads its inputs and writes its outputs.
 enum StageMode : int {
     SM_LDS = 0,    // LDS -> LDS, in place
     SM_FIRST = 1,  // the line's contiguous HBM elements -> LDS
     SM_LAST = 2,   // LDS -> the line's contiguous HBM elements (scaled)
+    SM_EXACT = 3,  // SM_LDS with the twiddles of table_powers
 };
 
 // One Stockham stage of the runtime-shape kernels. SM_LDS reads every input
@@ -416,7 +433,7 @@ __device__ __forceinline__ void stage_rt_body(cpx<T>* __restrict__ line, int N, 
             }
         }
     }
-    if constexpr (MODE == SM_LDS) __syncthreads();
+    if constexpr (MODE == SM_LDS || MODE == SM_EXACT) __syncthreads();
     const int step = N / (P * R);
 #pragma unroll
     for (int j = 0; j < MJ; ++j) {
@@ -425,7 +442,10 @@ __device__ __forceinline__ void stage_rt_body(cpx<T>* __restrict__ line, int N, 
             const int k = (int)((unsigned)b % (unsigned)P);
             if (P > 1) {
                 cpx<T> wp[R];
-                root_powers<R>(stage_root<T>(tw, k * step, P >= kScatterP), wp);
+                if constexpr (MODE == SM_EXACT)
+                    table_powers<R>(tw.full, k * step, wp);
+                else
+                    root_powers<R>(stage_root<T>(tw, k * step, P >= kScatterP), wp);
 #pragma unroll
                 for (int i = 1; i < R; ++i) v[j][i] = twmul<S>(v[j][i], wp[i]);
             }
@@ -520,7 +540,7 @@ __device__ __forceinline__ void stage_rt_radix(int R, cpx<T>* __restrict__ line,
     case RR: stage_rt<T, S, RR, WIDE, MODE>(line, N, P, TT, t, ps, tw, gsrc, gdst, valid, sc); break;
     switch (R) {
         case 2:
-            if constexpr (MODE == SM_LDS) stage_rt<T, S, 2, WIDE, MODE>(line, N, P, TT, t, ps, tw, gsrc, gdst, valid, sc);
+            if constexpr (MODE == SM_LDS || MODE == SM_EXACT) stage_rt<T, S, 2, WIDE, MODE>(line, N, P, TT, t, ps, tw, gsrc, gdst, valid, sc);
             break;
         VKFX_STAGE_CASE(3)
         VKFX_STAGE_CASE(4)
@@ -785,8 +805,8 @@ __device__ __noinline__ void stage_rader_fft(cpx<T>* __restrict__ line, cpx<T>* 
 // Runs every stage of a runtime radix list over the line at `line` (in LDS);
 // with RAD, a Rader stage (radix above kMaxStockhamRadix) uses `scr` and its
 // table block in `rtab` (RAD instantiations only, so the Rader stages'
-// registers stay out of the other kernels).
-template <typename T, int S, bool WIDE, bool RAD = false>
+// registers stay out of the other kernels). EXACT: twiddles of table_powers.
+template <typename T, int S, bool WIDE, bool RAD = false, bool EXACT = false>
 __device__ __forceinline__ void run_stages(cpx<T>* __restrict__ line, const int N, const int TT,
                                            const int t, const int ps, const int nst,
                                            const int* __restrict__ radix, const StageTw& tw,
@@ -795,7 +815,7 @@ __device__ __forceinline__ void run_stages(cpx<T>* __restrict__ line, const int 
     int P = 1;
     for (int s = 0; s < nst; ++s) {
         if (!RAD)
-            stage_rt_radix<T, S, WIDE, SM_LDS>(radix[s], line, N, P, TT, t, ps, tw, nullptr, nullptr, 0, (T)1);
+            stage_rt_radix<T, S, WIDE, EXACT ? SM_EXACT : SM_LDS>(radix[s], line, N, P, TT, t, ps, tw, nullptr, nullptr, 0, (T)1);
         else if (radix[s] > kMaxStockhamRadix && (roff[s] & kRaderFftStage))
             stage_rader_fft<T, S>(line, scr, N, P, radix[s], TT, t, ps, tw,
                                   (const unsigned char*)rtab + (roff[s] & ~kRaderFftStage));

@@ -16,6 +16,11 @@
 // 7.7, x 244 15.4 -> 9.8, x 1953 52.1 -> 45.0; 16 x 16 x 31250 69 -> 44; 63 x 65 15.9 -> 9.0;
 // 16^3 x 244 26.4 -> 10.2; 2 x 2000 x 250 35 -> 12; f64 30 x 14 x 2380 27.4 -> 15.7,
 // 4 x 1000 x 250 92.7 -> 14.1. Nontemporal accesses measured the same.
+//
+// Twiddles by table_powers: error against 64 bits, f32, products of one root -> these
+// loads, with the axis passes: 1000 x 2 x 2 2.19e-7 -> 1.29e-7 (1.57e-7), 80 x 60 1.65e-7
+// -> 1.28e-7 (1.50e-7), 3087 x 2 2.02e-7 -> 1.38e-7 (1.86e-7), at the same times (all
+// R - 1 roots from the table: 12 x 720 x 347 27.9 us against 26.6).
 #pragma once
 #include "fft_device.hpp"
 #include "kernels.hpp"
@@ -36,25 +41,6 @@ struct FieldDiv {
     __device__ __forceinline__ explicit FieldDiv(unsigned v) : m(v > 1 ? 0xffffffffu / v + 1 : 0), d(v) {}
     __device__ __forceinline__ int operator()(int x) const { return d > 1 ? (int)__umulhi((unsigned)x, m) : x; }
 };
-
-// p[i] = w^i, i < R, w = root `m` of the table: the powers of two from the table, the
-// others as products of them, at most three factors each rounded once. A tree of
-// products from w alone (root_powers) squares w's own rounding error up to the
-// eighth power; measured against 64 bits, f32, tree -> these loads, with the axis
-// passes: 1000 x 2 x 2 2.19e-7 -> 1.29e-7 (1.57e-7), 80 x 60 1.65e-7 -> 1.28e-7
-// (1.50e-7), 3087 x 2 2.02e-7 -> 1.38e-7 (1.86e-7), at the same times (all R - 1 roots
-// from the table: 12 x 720 x 347 27.9 us against 26.6).
-template <int R, typename T>
-__device__ __forceinline__ void field_roots_of(const void* tw, int m, cpx<T>* p) {
-#pragma unroll
-    for (int i = 1; i < R; i *= 2) p[i] = ld_table<T>(tw, i * m);
-#pragma unroll
-    for (int i = 3; i < R; ++i) {
-        int hb = 1;
-        while (hb * 2 <= i) hb *= 2;
-        if (hb != i) p[i] = cmul(p[i - hb], p[hb]);
-    }
-}
 
 // One radix-R stage of the axis of n points and stride `inner`, `elems`
 // elements in all, P the product of the axis's earlier radices.
@@ -90,7 +76,7 @@ __device__ __noinline__ void field_stage(const cpx<T>* src, cpx<T>* dst, int ele
         const int k = b - by_p(b) * P;
         if (P > 1) {
             cpx<T> wp[R];
-            field_roots_of<R>(tw, k * step, wp);
+            table_powers<R>(tw, k * step, wp);
 #pragma unroll
             for (int i = 1; i < R; ++i) v[i] = twmul<S>(v[i], wp[i]);
         }

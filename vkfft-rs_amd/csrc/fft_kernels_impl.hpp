@@ -808,6 +808,13 @@ struct IoC2RHalfEdge : IoC2RHalf {
 #include "fft_r2r.hpp"
 namespace vkfx {
 
+// Runtime-shape lines whose twiddles come from table_powers: the DCT / DST lines,
+// whose half-length FFTs with products of one root were further from 64 bits than
+// the full-length ones of the three passes they replace (f32 DCT-II columns 8192 x 64
+// 1.4 times).
+template <class IO>
+constexpr bool exact_tw = std::is_same_v<IO, IoR2rII> || std::is_same_v<IO, IoR2rIII> || std::is_same_v<IO, IoR2rMisc>;
+
 // Four-step column pass. Line = column n2 of the [N1][N2] view (C = N2);
 // FFT over n1 (length N1); store Y[k1][n2] * W_M^(dir * n2 * k1).
 struct IoFsA : IoPlain {
@@ -1613,7 +1620,7 @@ __global__ __launch_bounds__(512) void k_dyn(const KArgs a) {
     // Rader stages (radix > kMaxStockhamRadix) stage their inputs in a second
     // region of G lines after the lines themselves
     cpx<T>* scr = RAD ? lds + a.G * a.LS + g * a.LS : nullptr;
-    run_stages<T, S, WIDE, RAD>(line, a.N, a.TT, t, a.PS, a.nstages, a.radix, tw, scr, a.rtab, a.roff);
+    run_stages<T, S, WIDE, RAD, exact_tw<IO>>(line, a.N, a.TT, t, a.PS, a.nstages, a.radix, tw, scr, a.rtab, a.roff);
     if constexpr (IO::kTwoPass) {
         IO::template mid<T, DynDims>(a, lds, li);
         __syncthreads();

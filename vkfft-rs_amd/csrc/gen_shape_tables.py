@@ -854,7 +854,10 @@ def b(v):
 # 1.70e-7 from tables; 1080 x 1920 3.14e-7, 3.28e-7, 2.81e-7; f64 960 x 540 6.4e-16,
 # 7.0e-16, 6.2e-16), at the same times (1080 x 1920 x 4 58.7 us as products, 58.4 from
 # tables, 1024 x 1024 x 8 56.9 and 56.7; convolutions of one 1024 x 1024 f32 31.8 and 32.7).
-STAGE_TABLES = ("kf_cols_f32", "kf_cols_f64")
+# DCT / DST lines: f32 DST-II 8192 x 100 1.45 times the error of the three passes as
+# products, 0.48 times from tables; 16.0 and 16.4 us (three passes 46), f64 8192 x 100
+# 19.0 and 20.8 (48).
+STAGE_TABLES = ("kf_cols_f32", "kf_cols_f64", "kf_r2r_f32", "kf_r2r_f64")
 
 
 def render(name):
