@@ -16,14 +16,14 @@ constexpr size_t kStaticScratchBytes = size_t(64) << 20;
 constexpr int kMaxDevices = 64;
 hipError_t static_scratch_address(int device, void** out);
 
-// Kernel families. Each is one HBM pass over its lines; see the comments on
-// the IO policies in fft_kernels.hip for what each one loads and stores.
 #ifdef __HIPCC__
 #define VKFX_HD __host__ __device__
 #else
 #define VKFX_HD
 #endif
 
+// Kernel families. Each is one HBM pass over its lines; see the comments on
+// the IO policies in fft_kernels_impl.hpp for what each one loads and stores.
 enum KernelKind : int {
     KK_PLAIN = 0,      // C2C lines along any axis, scale on store
     KK_R2C_FULL,       // odd-length R2C: real -> complex FFT, keep n/2+1

@@ -1,6 +1,6 @@
 // runtime.cpp -- context, plans and the C ABI of the MI355X FFT path.
 //
-// A plan is a list of kernel launches (fft_kernels.hip) with their tables
+// A plan is a list of kernel launches (fft_kernels_impl.hpp) with their tables
 // (twiddles, chirps, kernel spectra) uploaded once at plan time, mirroring
 // what vkfft-rs's HIP runtime keeps in its module/LUT caches
 // (src/backend/hip/runtime.rs:1422-1468, 2019-2039) but without any source
@@ -1478,8 +1478,6 @@ bool shares_lines(size_t inner, int G, int prec, size_t len, size_t lines) {
     return (inner * csize(prec)) % 128 != 0 || ((size_t)G * csize(prec)) % 128 != 0;
 }
 
-// Axes whose bit is set in `omit` are left untransformed (the real axis of an
-// N-D real transform).
 // Stage radices of a field's axis: the fewest stages, and of those the smallest
 // sum of radices (stages cost a pass over LDS and a barrier each). wide: with
 // radices 12 and 16.
@@ -1643,6 +1641,8 @@ bool plan_field(Ctx& c, const vkfx_plan_desc& d, int* rc) {
     return true;
 }
 
+// Axes whose bit is set in `omit` are left untransformed (the real axis of an
+// N-D real transform).
 int plan_c2c_nd(Ctx& c, const vkfx_plan_desc& d, uint32_t omit) {
     const int prec = c.prec;
     const int dir = d.direction;
@@ -2292,10 +2292,14 @@ int plan_r2r(Ctx& c, size_t n, size_t batch, int kind, int dir, bool normalize, 
                                     planner_device(p->ctx->profile.shared_memory_bytes));
     p->serial = true;
     static const char* kNames[] = {"dct1", "dct2", "dct3", "dct4", "dst1", "dst2", "dst3", "dst4"};
-    c.js << "\"r2r\":{\"type\":\"" << kNames[kind] << "\",\"runs\":\"" << kNames[eff] << "\",\"fft_len\":" << L
-         << ",\"c2c\":\""
-         << (ad.algorithm == Algorithm::Stockham ? "stockham" : ad.algorithm == Algorithm::Rader ? "rader" : "bluestein")
-         << "\"},";
+    // fft_len: the complex FFT of the type's reduction; kernel_fft_len: the FFT that
+    // the launches run (half of it, packed, in most one-kernel lines)
+    auto describe = [&](size_t kernel_len) {
+        c.js << "\"r2r\":{\"type\":\"" << kNames[kind] << "\",\"runs\":\"" << kNames[eff] << "\",\"fft_len\":" << L
+             << ",\"kernel_fft_len\":" << kernel_len << ",\"c2c\":\""
+             << (ad.algorithm == Algorithm::Stockham ? "stockham" : ad.algorithm == Algorithm::Rader ? "rader" : "bluestein")
+             << "\"},";
+    };
     // One kernel per line where the packed (even types: half-length) FFT of
     // the reduction is a Stockham length of one upload; odd type IV, longer
     // lines and lines whose reduction runs as Rader or Bluestein keep the
@@ -2368,6 +2372,7 @@ int plan_r2r(Ctx& c, size_t n, size_t batch, int kind, int dir, bool normalize, 
             k.nvalid = (long long)n;
             k.rop = form;
             k.rflip = dst ? 1 : 0;
+            describe(N);
             // every phase lies in the first quarter of its circle; short lines' are exact
             // (as products of two levels f64 DCT-II 96 x 32 had 1.06 times the error of the
             // three passes, 0.99 to 1.01 this way)
@@ -2377,6 +2382,7 @@ int plan_r2r(Ctx& c, size_t n, size_t batch, int kind, int dir, bool normalize, 
                               0, "r2r_line");
         }
     }
+    describe(L);
     a.s *= scale;
     p->full_bytes = std::max(p->full_bytes, batch * L * csize(c.prec));
     Launch pre{};
