@@ -109,3 +109,52 @@ def test_mixed_storage(hip_ctx, prec, tol):
         xs = x.real.astype(np.float16).astype(np.float64) + 1j * x.imag.astype(np.float16).astype(np.float64)
     ref = np.fft.fft2(xs.astype(np.complex128).reshape(batch, n, inner), axes=(1, 2)).reshape(-1)
     assert o.rel_l2(y, ref) <= tol
+
+
+@pytest.mark.parametrize("prec,G", [(vk.Precision.F32, 16), (vk.Precision.F64, 8)])
+def test_every_convolution_length_is_fused(hip_ctx, prec, G):
+    """Every registered length's KK_CONV_1 shape, with a ragged last block (49
+    columns a tensor): three passes, the fixed shape in the middle."""
+    wide = prec == vk.Precision.F64
+    dt, inner = (np.complex128 if wide else np.complex64), 49
+    for n in LENGTHS:
+        batch = 97 * G // inner + 1
+        x = o.complex_uniform(n * inner * batch, n, dt)
+        k = o.complex_uniform(n * inner, n + 1, dt)
+        conv = vk.ConvolutionIr.build(vk.FftConfig.new([n, inner]).with_batch_count(batch).with_precision(prec), k)
+        plan = vk.Plan(hip_ctx, conv.ir, desc=conv.desc())
+        passes = plan.describe()["passes"]
+        plan.close()
+        assert [p["kernel"] for p in passes] == ["stockham_rows", "convolution_fused_axis0", "stockham_rows"], n
+        assert passes[1]["fixed_shape"] and passes[1]["lines_per_block"] == G and passes[1]["fft_len"] == n
+        y = hip_ctx.execute_convolution(conv, x)
+        X = np.fft.fftn(x.astype(np.complex128).reshape(batch, n, inner), axes=(1, 2))
+        ref = np.fft.ifftn(X * k.astype(np.complex128).reshape(n, inner), axes=(1, 2)).reshape(-1)
+        assert o.rel_l2(y, ref) <= (2e-13 if wide else 2e-6), n
+
+
+@pytest.mark.parametrize("prec,G,tol", [(vk.Precision.F16StorageF32Compute, 16, 1e-3),
+                                        (vk.Precision.F64ComputeF32Storage, 8, 1e-7)])
+def test_every_length_stores_half_precision(hip_ctx, prec, G, tol):
+    """Every registered length's KK_PLAIN_EDGE_OUT shape: no boundary pass, the
+    conversion inside the one pass over the columns (rows of 256, whose shape reads
+    half precision)."""
+    inner = 256
+    for n in LENGTHS:
+        batch = 97 * G // inner + 1
+        x = o.complex_uniform(n * inner * batch, n, np.complex64)
+        for direction, f in ((vk.Direction.Forward, np.fft.fft2), (vk.Direction.Inverse, np.fft.ifft2)):
+            c = vk.FftConfig.new([n, inner]).with_batch_count(batch).with_precision(prec).with_inverse_normalization(True)
+            ir = vk.TransformIr.build(c, direction)
+            d = hip_ctx.plan(ir).describe()
+            assert d["boundary"]["fused_edges"], n
+            assert [(p["kernel"], p["fixed_shape"]) for p in d["passes"]] == [("stockham_rows", True), ("stockham_columns", True)], n
+            assert d["passes"][1]["lines_per_block"] == G, n
+            y = hip_ctx.execute_transform_f32(ir, x)
+            xs = x
+            if prec == vk.Precision.F16StorageF32Compute:
+                xs = x.real.astype(np.float16).astype(np.float64) + 1j * x.imag.astype(np.float16).astype(np.float64)
+            ref = f(xs.astype(np.complex128).reshape(batch, n, inner), axes=(1, 2)).reshape(-1)
+            # inverses in binary16 are small numbers: their spacing is 2^-24 below 2^-14
+            slack = 2.0 ** -25 * np.sqrt(2 * ref.size) / np.linalg.norm(ref) if prec == vk.Precision.F16StorageF32Compute else 0.0
+            assert o.rel_l2(y, ref) <= tol + slack, (n, direction)

@@ -73,6 +73,69 @@ def test_strided_lines(hip_ctx, name, prec):
         _check(y, ref, n, prec)
 
 
+def _shapes(prec):
+    """(half length, lines a block, columns) of every registered type II / III shape."""
+    import importlib.util
+    import os
+    src = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "vkfft-rs_amd", "csrc", "gen_shape_tables.py")
+    spec = importlib.util.spec_from_file_location("gen_shape_tables", src)
+    g = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(g)
+    rows = g.TABLES["kf_r2r_f64" if prec == vk.Precision.F64 else "kf_r2r_f32"]
+    return sorted({(r[2], r[4], r[5]) for r in rows})
+
+
+@pytest.mark.parametrize("name", ["dct2", "dct3", "dst2", "dst3"])
+@pytest.mark.parametrize("col", [False, True])
+@pytest.mark.parametrize("prec", [vk.Precision.F32, vk.Precision.F64])
+def test_every_registered_shape(hip_ctx, name, col, prec):
+    """All fixed shapes of types II and III, rows and columns, one full block and a
+    ragged one (columns: over two outer lines, so that blocks cross them)."""
+    import scipy.fft as sf
+    f = sf.dct if name.startswith("dct") else sf.dst
+    dt = np.float32 if prec == vk.Precision.F32 else np.float64
+    seen, unreached = 0, []
+    for M, G, is_col in _shapes(prec):
+        if is_col != col:
+            continue
+        n, seen = 2 * M, seen + 1
+        dims, batch = ([n, G // 2 + 2], 2) if col else ([n], G + 1)
+        x = o.uniform(int(np.prod(dims)) * batch, n, dt)
+        ir = _plan(hip_ctx, name, dims, batch, prec, omit=(1,) if col else ())
+        plan = vk.Plan(hip_ctx, ir)
+        passes = plan.describe()["passes"]
+        plan.close()
+        if len(passes) != 1:
+            unreached.append(M)
+            continue
+        (p,) = passes
+        assert p["kernel"] == "r2r_line" and p["fixed_shape"] and p["lines_per_block"] == G and p["fft_len"] == M, (n, p)
+        y = hip_ctx.execute_transform(ir, x)
+        _check(y, f(x.astype(np.float64).reshape([batch] + dims), type=int(name[-1]), axis=1).reshape(-1), n, prec)
+    assert seen >= 60 and not unreached, unreached
+
+
+@pytest.mark.parametrize("name", KINDS)
+def test_described_lengths_are_the_executed_ones(hip_ctx, name):
+    """The description's kernel length is that of the launch: half of the reduction's
+    in the packed forms of types II and III, N -+ 1 in type I."""
+    t = int(name[-1])
+    for n in (64, 63):
+        ir = _plan(hip_ctx, name, [n], 2, vk.Precision.F32)
+        d = hip_ctx.plan(ir).describe()
+        kernel = d["r2r"]["kernel_fft_len"]
+        if t == 4 and n % 2:
+            assert kernel == d["r2r"]["fft_len"] == 2 * n and len(d["passes"]) > 1
+            continue
+        # DCT-I of 64 points: the even extension has 126, a Stockham length; of 63, 124 = 4 x 31 is none
+        if len(d["passes"]) == 1:
+            assert d["passes"][0]["kernel"] == "r2r_line" and d["passes"][0]["fft_len"] == kernel
+            assert kernel == {1: n - 1 if name == "dct1" else n + 1, 2: n // 2 if n % 2 == 0 else n,
+                              3: n // 2 if n % 2 == 0 else n, 4: n // 2}[t]
+        else:
+            assert kernel == d["r2r"]["fft_len"] and t == 1
+
+
 @pytest.mark.parametrize("name", KINDS)
 @pytest.mark.parametrize("prec", [vk.Precision.F32, vk.Precision.F64])
 def test_few_lines(hip_ctx, name, prec):

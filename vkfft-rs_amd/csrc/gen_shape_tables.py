@@ -737,6 +737,10 @@ def r2r_rows(prec):
 
     for m in sorted(src):
         _, _, _, tt, G, _, rad, ps, ls = src[m]
+        # a plan takes one kernel where the runtime shapes hold the line too: 512
+        # threads of 32 elements a stage (16000 points in radices of 10 need 534)
+        if any(-(-(m // r) // (32 // r)) > 512 for r in rad):
+            continue
         small = radix_plan(m, (8, 6, 5, 4, 3, 2))
         if small and (prec or (max(rad) == 16 and m & (m - 1))):
             rad = small
