@@ -10,9 +10,10 @@
 // block's elements, so that adjacent lanes touch adjacent elements on every
 // axis.
 //
-// Single fields are bound by the chain of launches and stages, batches of them
-// by LDS latency at 8 to 16 waves a CU (8M f32 points of 64 x 64: 128 MB in 45 us,
-// 2.8 TB/s). Measured, us a pass, axis passes -> one kernel: f32 64 x 64 8.8 ->
+// Bound by the latency of the chain of stages (a table load, an LDS round trip and a
+// barrier each) at 8 to 16 waves a CU: waves wait 63 to 70% of their cycles and issue
+// VALU work in 12 to 14% (f32 64 x 64 x 244, f64 16^3 x 244); 8M f32 points of 64 x 64,
+// 128 MB, take 45 us, 2.8 TB/s. Measured, us a pass, axis passes -> one kernel: f32 64 x 64 8.8 ->
 // 7.7, x 244 15.4 -> 9.8, x 1953 52.1 -> 45.0; 16 x 16 x 31250 69 -> 44; 63 x 65 15.9 -> 9.0;
 // 16^3 x 244 26.4 -> 10.2; 2 x 2000 x 250 35 -> 12; f64 30 x 14 x 2380 27.4 -> 15.7,
 // 4 x 1000 x 250 92.7 -> 14.1. Nontemporal accesses measured the same.

@@ -13,15 +13,15 @@
 // Bound by HBM: 8 bytes of traffic a real (f32) in one pass, against a pre
 // pass, a full-length complex FFT and a post pass (40 bytes a real, with the
 // phases from sincospi and strided gathers). f32 DCT-II and its normalized
-// inverse over 16 x 720 x 1280: 1016 us in 12 launches before, 125 us in 4 (31-34
-// us a pass over 118 MB, 3.5-3.8 TB/s), with the error against 64 bits at 3.1e-7
+// inverse over 16 x 720 x 1280: 1020 us in 12 launches before, 131 us in 4 (32-36
+// us a pass over 118 MB, 3.3-3.5 TB/s), with the error against 64 bits at 2.2e-7
 // from 3.9e-7. The first version, with block-wide copies whose loads wait one at a
 // time and a table lookup per phase, ran 276 us.
 #pragma once
 
 namespace vkfx {
 
-// exp(-2 pi i k / L) of the launch's two-level f64 phase table
+// exp(-2 pi i k / L) of the launch's f64 phase table (one level for short lines)
 __device__ __forceinline__ cpx<double> r2r_root(const KArgs& a, long long k) {
     return tw2<double>(a.rlo, a.rhi, a.rshift, k);
 }

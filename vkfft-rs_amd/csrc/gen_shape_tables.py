@@ -778,7 +778,7 @@ HEADS_R2R = ("// Fixed shapes of the one-kernel DCT / DST lines of types II and 
 HEADS['kf_r2r_f32'] = HEADS_R2R.format(p='f32')
 HEADS['kf_r2r_f64'] = HEADS_R2R.format(p='f64')
 
-# Strided axes longer than 640 points in one pass: 16 (f32) / 8 (f64) adjacent
+# Strided axes of 640 to 1247 points in one pass: 16 (f32) / 8 (f64) adjacent
 # lines (128-byte segments) in one block per CU, up to the length whose lines
 # fill the LDS. The radix plan's threads: of 32 to 64 threads a line, the fewest with
 # the fewest elements to handle one after another (a stage gives a thread
