@@ -4,7 +4,7 @@
 #include "fft_field.hpp"
 
 namespace vkfx {
-// radices up to 10 in 130 to 152 registers, larger ones (212) apart
+// radices up to 10 in 120 to 148 registers, larger ones (214) apart
 KernelFn pick_field_f64(int dir, bool large) {
     if (large) return dir < 0 ? k_field<double, -1, 16> : k_field<double, 1, 16>;
     return dir < 0 ? k_field<double, -1, 10> : k_field<double, 1, 10>;
