@@ -51,7 +51,8 @@ ALONE = [([20, 20, 20], 1, "f32", False), ([16, 16, 16], 1, "f64", True), ([12, 
          ([8, 512], 1, "f64", False), ([8, 512], 3, "f64", True), ([8, 512], 4, "f64", False), ([8, 512], 256, "f64", True), ([45, 64], 1, "f64", False),
          ([48, 108], 1, "f32", True), ([100, 80], 1, "f32", True), ([160, 50], 1, "f32", False), ([160, 50], 256, "f32", True),
          ([1000, 8], 1, "f32", False), ([270, 30], 256, "f32", False), ([80, 60], 513, "f32", False), ([91, 77], 57, "f32", True),
-         ([4, 2000], 31, "f32", False), ([4, 2000], 32, "f32", True), ([9, 792], 1, "f32", False), ([1024, 4], 1, "f64", True), ([2, 2, 1000], 1, "f64", True)]
+         ([4, 2000], 31, "f32", False), ([4, 2000], 32, "f32", True), ([9, 792], 1, "f32", False), ([48, 98], 63, "f32", False),
+         ([48, 98], 64, "f32", True), ([36, 105], 255, "f64", True), ([1024, 4], 1, "f64", True), ([2, 2, 1000], 1, "f64", True)]
 
 
 @pytest.mark.parametrize("dims,batch,prec,one", ALONE)

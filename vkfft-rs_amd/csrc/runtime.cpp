@@ -1534,7 +1534,9 @@ FieldWanted field_wanted() {
 // field_slow, for fields alone on a CU: `trips` is the sum over the stages of the
 // butterflies a thread runs one after another (about 0.7 us each beside 5 us);
 // `quick`: every strided axis is on a fixed shape or on a runtime shape nearly as
-// fast (12 points and more without the factors 7, 11 and 13). us, axis passes
+// fast (12 points and more without the factors 7, 11 and 13), and the rows lack those
+// factors or the fields are few (below 64: 6 x 819 x 40 f32 10.0 against 10.7; more: 36 x
+// 105 x 255 f64 23.4 against 14.3, 48 x 98 x 445 f32 33.1 against 23.1). us, axis passes
 // against one kernel:
 // - fewer blocks than CUs, 3-D: 20^3 11.5 against 17.5 (24 trips), 30 x 30 x 9 13.1
 //   against 15.6 (16), f64 12 x 12 x 20 11.2 against 12.3 (14), 16^3 14.3 against 8.5 (3);
@@ -1580,7 +1582,7 @@ bool plan_field(Ctx& c, const vkfx_plan_desc& d, int* rc) {
         const bool five = n % 7 && n % 11 && n % 13;
         fixed &= has;
         smooth &= five;
-        quick &= has || last || (five && n >= 12);
+        quick &= has || (last ? five || d.batch < 64 : five && n >= 12);
     }
     auto buffers = [&](size_t points) { return 2 * ((points + (points >> 3) + 2) / 2 * 2); };
     if (buffers(total) * cs > std::min<size_t>(c.lds_max, 156 * 1024)) return false;
