@@ -39,8 +39,9 @@ def test_strided_passes(hip_ctx, dims, batch, prec):
                                                ([24, 405], 540, True), ([127, 405], 2, False), ([128, 405], 2, True),
                                                ([24, 400], 540, False), ([200, 120], 4, False)])
 def test_rule_by_size(hip_ctx, dims, batch, shared):
-    """Short lines and pitches of half memory lines keep the round-robin order and nontemporal stores from 512 KB
-    to 40 MB, and everywhere where the row pitch is whole memory lines."""
+    """A last pass over short lines or pitches of half memory lines keeps the round-robin
+    order and nontemporal stores from 512 KB to 40 MB, and everywhere where the row
+    pitch is whole memory lines."""
     x = o.complex_uniform(int(np.prod(dims)) * batch, 3, np.complex64)
     ir = vk.TransformIr.build(vk.FftConfig.new(dims).with_batch_count(batch), vk.Direction.Forward)
     y = hip_ctx.execute_transform(ir, x)
@@ -50,3 +51,25 @@ def test_rule_by_size(hip_ctx, dims, batch, shared):
     assert p["xcd_groups"] == shared, p
     if p["fixed_shape"]:
         assert p["nontemporal"] == [False, not shared], p
+
+
+def test_passes_before_the_last_keep_their_ranges(hip_ctx):
+    """Sizes whose last pass streams: the middle axis of a volume, the columns of a
+    C2R, which the rows read next, and those of an R2C are dealt in ranges."""
+    dims, batch = [40, 40, 45], 4
+    x = o.complex_uniform(int(np.prod(dims)) * batch, 3, np.complex64)
+    ir = vk.TransformIr.build(vk.FftConfig.new(dims).with_batch_count(batch), vk.Direction.Forward)
+    y = hip_ctx.execute_transform(ir, x)
+    ref = np.fft.fftn(x.astype(np.complex128).reshape([batch] + dims), axes=(1, 2, 3)).reshape(-1)
+    assert o.rel_l2(y, ref) <= 2e-6
+    passes = hip_ctx.plan(ir).describe()["passes"]
+    assert [(p["kernel"], p["xcd_groups"]) for p in passes] == [("stockham_rows", False), ("stockham_columns", True),
+                                                                ("stockham_columns", False)]
+    c = vk.FftConfig.new([60, 90]).with_batch_count(40).with_transform(vk.TransformKind.ComplexToReal)
+    names = [(p["kernel"], p["xcd_groups"]) for p in
+             hip_ctx.plan(vk.TransformIr.build(c, vk.Direction.Inverse)).describe()["passes"]]
+    assert names == [("stockham_columns", True), ("c2r_even_half", False)]
+    c = vk.FftConfig.new([60, 90]).with_batch_count(40).with_transform(vk.TransformKind.RealToComplex)
+    names = [(p["kernel"], p["xcd_groups"]) for p in
+             hip_ctx.plan(vk.TransformIr.build(c, vk.Direction.Forward)).describe()["passes"]]
+    assert names == [("r2c_even_half", False), ("stockham_columns", True)]

@@ -1459,23 +1459,30 @@ bool split_strided_axis(const Ctx& c, size_t len, size_t lines, size_t* l1, size
 // ranges). Measured, us a pass, round-robin and nontemporal against ranges and
 // cached: f32 columns of 512 over rows of 405 36.2 -> 23.8, 360 27.4 -> 18.5,
 // 100 20.6 -> 14.5, 1080 over 961 (16 frames, inverse) 87 -> 63; f64 512 over 405
-// 29.8 -> 25.5; [405, 405, 75] x 2 whole 349 -> 256. Passes of 512 KB to 40 MB over
-// lines shorter than 128, or whose row pitch is whole halves of memory lines, keep the round-robin order and the nontemporal stores:
-// most of their output waits in the 32 MB of L2 for the end of the kernel, and is
-// written back then. Whole transforms, round-robin against ranges, lines of 18 to
-// 100 over rows of 60 to 961: 16 MB 1.00 to 1.12 times as long in ranges (24 x 405 x 215
-// f32 1.10, 128 x 60 x 136 f64 1.08), 64 MB 0.82 to 1.00; lines of 128 and 360 16 MB 0.85
-// to 1.06, 64 MB 0.73 to 0.98; below 512 KB ranges take 0 to 0.9 us more of 8 to 14
-// (30^3 f32 13.7 against 14.5) and 0.6 less (320 x 1001).
-// The passes of a split axis keep
+// 29.8 -> 25.5; [405, 405, 75] x 2 whole 349 -> 256; runtime shapes of 5 columns, 184 x
+// 128 x 8 whole 23.9 -> 21.4. The passes of a split axis keep
 // their order: the first (segments along L2 x inner) measured 5-15% slower in
 // ranges, the second 3-10% faster on its own, but the pass that follows it slower
 // by as much (1080 x 1920 frames, inverse: 49 -> 52 and C2R rows 56 -> 65).
-bool shares_lines(size_t inner, int G, int prec, size_t len, size_t lines) {
-    const size_t bytes = len * lines * csize(prec);
-    const bool halves = (inner * csize(prec)) % 64 == 0;
-    if ((len < 128 || halves) && bytes >= (512u << 10) && bytes < (40u << 20)) return false;
+bool shares_lines(size_t inner, int G, int prec) {
     return (inner * csize(prec)) % 128 != 0 || ((size_t)G * csize(prec)) % 128 != 0;
+}
+
+// A C2C plan's last pass over such lines, of 512 KB to 40 MB, whose lines are shorter
+// than 128 or whose rows and blocks are whole halves of memory lines, keeps the
+// round-robin order and the nontemporal stores: nothing reads its output again, and
+// most of it would wait in the 32 MB of L2 for the end of the kernel to be written
+// back. Whole 2-D transforms, round-robin against ranges, lines of 18 to 100 over rows
+// of 60 to 961: 16 MB 1.00 to 1.12 times as long in ranges (24 x 405 x 215 f32 1.10, 128 x
+// 60 x 136 f64 1.08), 64 MB 0.82 to 1.00; lines of 128 and 360 16 MB 0.85 to 1.06, 64 MB
+// 0.73 to 0.98; below 512 KB ranges take 0 to 0.9 us more of 8 to 14 (30^3 f32 13.7
+// against 14.5) and 0.6 less (320 x 1001). Passes whose output is read next gain from
+// ranges at every size, the last one of an R2C too (real pairs 117 x 81 x 256 81.8 ->
+// 73.7, 27 x 32 x 6526 66.3 -> 60.7).
+bool streams_last_pass(const KArgs& a, int prec) {
+    const size_t cs = csize(prec), bytes = (size_t)a.N * (size_t)a.nlines * cs;
+    const bool halves = ((size_t)a.C * cs) % 64 == 0 && ((size_t)a.G * cs) % 64 == 0;
+    return (a.N < 128 || halves) && bytes >= (512u << 10) && bytes < (40u << 20);
 }
 
 // Stage radices of a field's axis: the fewest stages, and of those the smallest
@@ -1744,7 +1751,7 @@ int plan_c2c_nd(Ctx& c, const vkfx_plan_desc& d, uint32_t omit) {
                             "N-D axis length " + std::to_string(len) + " exceeds one upload");
             const int want = contiguous ? std::max(1, 256 / g0.TT) : (prec ? 8 : 16);
             Geometry g = kernel_geometry(KK_PLAIN, prec, dir, len, !contiguous, want, c.lds_max, c.lds_budget);
-            if (!contiguous && shares_lines(inner, g.G, prec, len, (size_t)lines)) a.flags |= KF_XCD_GROUPS;
+            if (!contiguous && shares_lines(inner, g.G, prec)) a.flags |= KF_XCD_GROUPS;
             rc = add_launch(c, KK_PLAIN, dir, g, a, lines, blocks_for(lines, g.G), in_sel, off, SEL_OUT, off,
                             contiguous ? "stockham_rows" : "stockham_columns");
         } else {
@@ -1759,7 +1766,7 @@ int plan_c2c_nd(Ctx& c, const vkfx_plan_desc& d, uint32_t omit) {
                 if (g0.ok) {
                     const int want = contiguous ? std::max(1, 256 / g0.TT) : (prec ? 8 : 16);
                     Geometry g = geometry_rader(len, prec, want, c.lds_max, c.lds_budget);
-                    if (!contiguous && shares_lines(inner, g.G, prec, len, (size_t)lines)) a.flags |= KF_XCD_GROUPS;
+                    if (!contiguous && shares_lines(inner, g.G, prec)) a.flags |= KF_XCD_GROUPS;
                     note_rader_mixed(c, len, g);
                     return add_launch(c, KK_PLAIN, dir, g, a, lines, blocks_for(lines, g.G), in_sel, off, SEL_OUT,
                                       off, "rader_mixed_axis");
@@ -1776,7 +1783,7 @@ int plan_c2c_nd(Ctx& c, const vkfx_plan_desc& d, uint32_t omit) {
             if (rc) return rc;
             a.chirp = t.chirp, a.spec = t.spec;
             a.nvalid = (long long)len, a.nout = (long long)len, a.M = (long long)M;
-            if (!contiguous && shares_lines(inner, g.G, prec, len, (size_t)lines)) a.flags |= KF_XCD_GROUPS;
+            if (!contiguous && shares_lines(inner, g.G, prec)) a.flags |= KF_XCD_GROUPS;
             rc = add_launch(c, KK_BLUE_1, -1, g, a, lines, blocks_for(lines, g.G), in_sel, off, SEL_OUT, off,
                             "bluestein_axis");
         }
@@ -2204,7 +2211,7 @@ int plan_convolution(Ctx& c, const vkfx_plan_desc& d, size_t coords, size_t out_
             a.flags = (ca.conj_seq ? KF_CONV_CONJ : 0) | (ca.cross_norm ? KF_CONV_CROSS : 0);
             a.scale = 1.0 / (double)n0;
             a.spec = kernel;
-            if (shares_lines(rest, g.G, c.prec, n0, d.batch * rest)) a.flags |= KF_XCD_GROUPS;
+            if (shares_lines(rest, g.G, c.prec)) a.flags |= KF_XCD_GROUPS;
             const long long lines = (long long)(d.batch * rest);
             rc = add_launch(c, KK_CONV_1, -1, g, a, lines, blocks_for(lines, g.G), SEL_FULL, 0, SEL_OUT, 0,
                             "convolution_fused_axis0");
@@ -3429,6 +3436,8 @@ int vkfx_plan_create(vkfx_context* ctx, const vkfx_plan_desc* desc_in, vkfx_plan
     // registered variant.
     const char* ne = getenv("VKFX_NT_ROLES");
     const bool nt_roles = !(ne && ne[0] == '0');
+    const char* xe = getenv("VKFX_XCD_GROUPS");
+    const bool xcd_forced = xe && xe[0] == '1';
     for (size_t i = 0; nt_roles && i < p->launches.size(); ++i) {
         Launch& L = p->launches[i];
         if (!L.fixed) continue;
@@ -3436,8 +3445,13 @@ int vkfx_plan_create(vkfx_context* ctx, const vkfx_plan_desc* desc_in, vkfx_plan
         for (size_t j = i + 1; j < p->launches.size() && last; ++j) last = p->launches[j].chunk != L.chunk;
         // strided lines that share memory lines with their neighbours (shares_lines)
         if (L.kind == KK_PLAIN && L.fixed->col && (L.a.flags & KF_XCD_GROUPS)) {
-            L.fixed = fixed_variant(L.fixed, false, false);
-            continue;
+            if (last && L.out_sel == SEL_OUT && d.transform == VKFX_C2C && !d.perform_convolution && !xcd_forced &&
+                streams_last_pass(L.a, c.prec)) {
+                L.a.flags &= ~KF_XCD_GROUPS;
+            } else {
+                L.fixed = fixed_variant(L.fixed, false, false);
+                continue;
+            }
         }
         L.fixed = fixed_variant(L.fixed, L.in_sel == SEL_IN, L.out_sel == SEL_OUT && last);
     }
